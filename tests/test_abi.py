@@ -9,6 +9,7 @@ import ctypes
 import re
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 from kernelcode_generate_amd import native
@@ -89,3 +90,27 @@ def test_mfma_rate_probe_rejects_bad_arguments():
     assert rate(6, 32, 0, 0, 4, ctypes.byref(tf), ctypes.byref(ghz)) == -1
     assert rate(6, 16, 0, 10, 1 << 17, ctypes.byref(tf), ctypes.byref(ghz)) == -1
     assert not hasattr(native.load_library(), "kg_gfx950_mfma_rate")
+
+def test_packed_slots_hold_every_argument_kind():
+    """The words call_entry passes by address read back, through the C structure, as the
+    arguments: a strided view, a rank-0 tensor, an absent memory slot, integers beyond 32 and
+    (wrapped, as a C long long) 64 bits, numpy scalars and a float."""
+
+    import torch
+
+    view = torch.arange(60, dtype=torch.float16).reshape(3, 4, 5)[:, 1:3, ::2]
+    scalar = torch.tensor(2.0, dtype=torch.bfloat16)
+    args = (view, scalar, None, 1 << 40, -7, (1 << 64) + 3, np.int32(9), np.float32(0.5), -0.25)
+    slots, keep = native.marshal_slots(args)
+    assert len(slots) == len(args) and ctypes.sizeof(slots) == 64 * len(args)
+    kinds = [native.KG_ARG_MEMORY] * 3 + [native.KG_ARG_INT] * 4 + [native.KG_ARG_FLOAT] * 2
+    assert [s.kind for s in slots] == kinds
+    assert slots[0].data == view.data_ptr() and slots[0].rank == 3 and slots[0].dtype_code == 5
+    assert slots[0].shape[:3] == [3, 2, 3] and slots[0].stride[:3] == [20, 5, 2]
+    assert slots[1].data == scalar.data_ptr() and slots[1].rank == 0 and slots[1].dtype_code == 6
+    assert not slots[2].data and slots[2].rank == 1 and slots[2].shape[0] == 0 and slots[2].stride[0] == 1
+    assert [s.int_value for s in slots[3:7]] == [1 << 40, -7, 3, 9]
+    assert [s.float_value for s in slots[7:]] == [0.5, -0.25]
+    with pytest.raises(native.NativeLibraryError, match="unsupported runtime arg at position 1: str"):
+        native.marshal_slots((1, "x"))
+    del keep
