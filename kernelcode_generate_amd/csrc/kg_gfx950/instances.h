@@ -7,6 +7,7 @@
 
 #include "conv2d_igemm.h"
 #include "conv2d_mfma.h"
+#include "conv2d_nhwc.h"
 #include "conv2d_rowvec.h"
 #include "flash_attn_mfma.h"
 #include "gemm.h"
@@ -123,6 +124,16 @@ KG_IGEMM_INSTANCE(F16Tag, 2)
 KG_IGEMM_INSTANCE(F16Tag, 3)
 KG_IGEMM_INSTANCE(F16Tag, 4)
 #undef KG_IGEMM_INSTANCE
+#endif
+
+#if !defined(KG_INSTANTIATE) || defined(KG_INSTANTIATE_CONV_NHWC)
+#define KG_NHWC_INSTANCE(TAG)                                                                                     \
+  KG_INSTANCE hipError_t launch_conv2d_nhwc<TAG>(const void*, const void*, void*, const void*, int, const ConvShape&, \
+                                                 const ConvNhwcPlan&, char*, hipStream_t);
+KG_NHWC_INSTANCE(F32Tag)
+KG_NHWC_INSTANCE(Bf16Tag)
+KG_NHWC_INSTANCE(F16Tag)
+#undef KG_NHWC_INSTANCE
 #endif
 
 }  // namespace kg_gfx950

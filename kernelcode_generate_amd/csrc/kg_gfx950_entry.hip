@@ -23,6 +23,7 @@
 #include "kg_gfx950/gemm_f32.h"
 #include "kg_gfx950/conv2d_mfma.h"
 #include "kg_gfx950/conv2d_igemm.h"
+#include "kg_gfx950/conv2d_nhwc.h"
 #include "kg_gfx950/conv2d_rowvec.h"
 #include "kg_gfx950/flash_attn_mfma.h"
 #include "kg_gfx950/flash_attn_f32.h"
@@ -275,10 +276,11 @@ int pipe_splits(long long M, long long N, long long K, long long* chunk) {
   return (int)cdiv(K, c);
 }
 
-// Split-K workspaces, one per (device, stream) and kept for the life of the process: work
-// enqueued on one stream runs in order, so its calls can share one buffer, and calls on
-// different streams never do. A split call enqueues two kernels (the partial sums, then
-// their reduction), and a call holds its slot's lock (the lease) from the lookup until both
+// Workspaces (split-K partial sums; the channel-last conv's copy of its images and weights),
+// one per (device, stream) and kept for the life of the process: work enqueued on one stream
+// runs in order, so its calls can share one buffer, and calls on different streams never do.
+// Such a call enqueues two or more kernels (the partial sums or the copy, then their reader),
+// and a call holds its slot's lock (the lease) from the lookup until both
 // are enqueued: two host threads on one stream (every thread's default is the null stream)
 // therefore enqueue whole pairs, never A's partials, B's partials, A's reduction. A larger
 // request replaces the buffer (the old one is released in stream order, after the work
@@ -305,6 +307,17 @@ struct SplitLease {
 std::mutex g_split_ws_mutex;
 std::vector<SplitWorkspace> g_split_ws;
 unsigned long long g_split_ws_clock = 0;
+
+// True while the calling thread's stream records a graph (or cannot be asked because another
+// stream does).
+bool stream_capturing() {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(g_stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
 
 SplitLease split_workspace(size_t bytes, hipStream_t stream) {
   SplitLease lease;
@@ -646,11 +659,16 @@ int conv2d_impl(const KgArgSlot* args, unsigned long long n) {
                 out.shape[2], out.shape[3], x.shape[0], w.shape[0], ho, wo);
   if (bias.present && bias.shape[0] != w.shape[0]) return fail(kInvalid, "conv2d: bias extent != F");
   if (g_cost) {
-    long long mfma = 0;
+    const bool f32 = out.dtype == KG_DTYPE_F32;
+    long long mfma = 0, cyc = f32 ? 64 : 32;
+    const ConvNhwcPlan plan = conv_nhwc_plan(s, f32, kSplitMaxWorkspace);
     if (!staged && out.dtype != KG_DTYPE_F32 && conv_mfma_supported(s)) {  // live waves x 252 MFMAs per 7-row block
       mfma = (long long)s.n * ((s.h + convk::kRows - 1) / convk::kRows) * (s.w > 32 ? 4 : 2) * 252;
     } else if (conv_rowvec_supported(s, out.dtype == KG_DTYPE_F32)) {
       mfma = conv_rowvec_mfma(s, out.dtype == KG_DTYPE_F32);
+    } else if (plan.ok && !staged) {
+      mfma = conv_nhwc_mfma(s, plan, f32);  // 16x16x32, fp32 16x16x4
+      cyc /= 2;
     } else if (conv_igemm_supported(s)) {
       // implicit GEMM: per tile and 64-byte k slice, 4 waves x MI x 2 blocks x (2 MFMAs of
       // 32x32x16, or 8 of 32x32x2 for fp32)
@@ -660,7 +678,7 @@ int conv2d_impl(const KgArgSlot* args, unsigned long long n) {
       mfma = tiles * cdiv(K, bk) * 4 * mi * 2 * per;
     }
     const long long es = esize(out.dtype);
-    return record_cost(out.numel() * w.shape[1] * w.shape[2] * w.shape[3], mfma, out.dtype == KG_DTYPE_F32 ? 64 : 32,
+    return record_cost(out.numel() * w.shape[1] * w.shape[2] * w.shape[3], mfma, cyc,
                        (x.numel() + w.numel()) * es + (bias.present ? bias.shape[0] * esize(bias.dtype) : 0),
                        out.numel() * es);
   }
@@ -723,6 +741,25 @@ int conv2d_impl(const KgArgSlot* args, unsigned long long n) {
                                                       (int)stages);
     if (e != hipSuccess) return fail(kHipFailure, "conv2d(rowvec): %s", hipGetErrorString(e));
     return finish_launch("conv2d(rowvec)");
+  }
+  // Everything else: the channel-last copy and its GEMM, or, for tiny calls, a set stage count
+  // (that kernel's ring is its own), while a graph records (its workspace may be replaced
+  // later) and where the copy does not fit the workspace, the gathering implicit GEMM.
+  if (const ConvNhwcPlan plan = conv_nhwc_plan(s, out.dtype == KG_DTYPE_F32, kSplitMaxWorkspace);
+      plan.ok && !staged && aligned16(out.data) && !stream_capturing()) {
+    lease = split_workspace(plan.bytes(), g_stream);
+    if (char* ws = static_cast<char*>(lease.ptr)) {
+      const int bias_kind = !bias.present ? 0 : (bias.dtype == KG_DTYPE_F32 ? 1 : 2);
+      const void* bp = bias.present ? bias.data : nullptr;
+      hipError_t e =
+          out.dtype == KG_DTYPE_F32
+              ? launch_conv2d_nhwc<F32Tag>(x.data, w.data, out.data, bp, bias_kind, s, plan, ws, g_stream)
+          : out.dtype == KG_DTYPE_BF16
+              ? launch_conv2d_nhwc<Bf16Tag>(x.data, w.data, out.data, bp, bias_kind, s, plan, ws, g_stream)
+              : launch_conv2d_nhwc<F16Tag>(x.data, w.data, out.data, bp, bias_kind, s, plan, ws, g_stream);
+      if (e != hipSuccess) return fail(kHipFailure, "conv2d(nhwc): %s", hipGetErrorString(e));
+      return finish_launch("conv2d(nhwc)");
+    }
   }
   if (conv_igemm_supported(s) && aligned16(out.data)) {
     const int bias_kind = !bias.present ? 0 : (bias.dtype == KG_DTYPE_F32 ? 1 : 2);

@@ -316,3 +316,65 @@ def test_rejects_bad_params(device):
         native.conv2d(o, x, w, None, (0, 1), (1, 1), (1, 1, 1, 1))
     with pytest.raises(native.NativeLibraryError):
         native.conv2d(o, x, w, None, (1, 1), (1, 1), (0, 0, 0, 0))  # out shape mismatch
+
+
+@pytest.mark.parametrize("dtype_name", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize(
+    "xs,ws,stride,dil,pad,bias",
+    [
+        ((6, 20, 73, 71), (70, 20, 3, 3), (1, 1), (1, 1), (1, 1, 1, 1), "f32"),  # runs of 72 values, Ho Wo odd
+        ((8, 3, 121, 115), (53, 3, 7, 7), (2, 2), (1, 1), (3, 3, 3, 3), "same"),  # paired pixels, rows end mid-chunk
+        ((9, 4, 80, 90), (70, 4, 7, 4), (2, 2), (1, 1), (3, 3, 2, 1), None),  # paired pixels, even KW
+        ((4, 3, 101, 95), (53, 3, 7, 7), (1, 1), (1, 1), (3, 3, 3, 3), "f32"),  # 3 channels, stride 1
+        ((8, 17, 30, 33), (65, 17, 3, 3), (1, 1), (2, 2), (2, 2, 2, 2), "same"),  # dilated: runs are taps
+        ((2, 130, 29, 29), (129, 130, 3, 3), (2, 1), (1, 2), (1, 0, 2, 1), "f32"),  # dilated columns, ragged everywhere
+        ((9, 390, 21, 23), (72, 390, 1, 1), (1, 1), (1, 1), (0, 0, 0, 0), None),  # one tap
+        ((9, 24, 80, 91), (70, 24, 5, 1), (1, 2), (1, 1), (2, 2, 0, 0), "f32"),  # an odd number of halves
+        ((2, 300, 15, 15), (64, 300, 3, 3), (1, 1), (1, 1), (1, 1, 1, 1), "same"),  # K split
+        ((9, 24, 61, 63), (200, 24, 3, 3), (1, 1), (1, 1), (1, 1, 1, 1), None),  # 128-pixel tiles
+        ((8, 3, 112, 111), (192, 3, 7, 7), (2, 2), (1, 1), (3, 3, 3, 3), "f32"),  # 128-pixel tiles, short K
+        ((6, 64, 301, 301), (8, 64, 3, 3), (1, 1), (1, 1), (1, 1, 1, 1), "same"),  # several passes over the batch
+    ],
+    ids=["c20", "paired7", "paired4", "c3s1", "dil2", "dilw2", "tap1", "halves5", "split", "bm128", "bm128_shortk", "passes"],
+)
+def test_channel_last_matches_gather(device, dtype_name, xs, ws, stride, dil, pad, bias):
+    """The channel-last form against the gathering implicit GEMM (which a call that sets its
+    LDS stage count takes) on the same inputs. Both sum the same products in fp32 in another
+    order and round once: 16-bit outputs differ by at most one spacing of the format (8 and 11
+    significand bits: 2^-7 and 2^-10 of the value at a power of two, half a spacing for each
+    side's rounding; f16 below its normal range 2^-24) plus, as fp32 ones, twice the
+    rounding of a K-term sum, 4 sqrt(K) 2^-24 (|W| * |X|) (Higham and Mary, SIAM J. Sci. Comput. 41
+    (2019)). A second run with infinities in the image: a window that does not hold one must
+    not meet it in the padding of a run."""
+
+    import torch
+
+    dt = getattr(torch, dtype_name)
+    gen = torch.Generator(device=device).manual_seed(sum(xs) + sum(ws))
+    k = ws[1] * ws[2] * ws[3]
+    x = torch.randn(xs, generator=gen, device=device).to(dt)
+    w = ((torch.rand(ws, generator=gen, device=device) * 2 - 1) * (6.0 / k) ** 0.5).to(dt)
+    b = None if bias is None else torch.randn(ws[0], generator=gen, device=device)
+    if bias == "same":
+        b = b.to(dt)
+    ho = (xs[2] + pad[0] + pad[1] - dil[0] * (ws[2] - 1) - 1) // stride[0] + 1
+    wo = (xs[3] + pad[2] + pad[3] - dil[1] * (ws[3] - 1) - 1) // stride[1] + 1
+    specs = [native.TensorSpec(s, dtype_name) for s in ((xs[0], ws[0], ho, wo), xs, ws)]
+    model = native.cost("conv2d", [*specs, None, *stride, *dil, *pad])
+    assert model["MFMA_CYCLES"] == model["MFMA"] * (32 if dt == torch.float32 else 16)  # the route under test
+
+    def conv(xt, wt, bt, stage):
+        out = torch.full((xs[0], ws[0], ho, wo), float("nan"), dtype=dt, device=device)
+        print(f"[conv2d] channel-last {dtype_name} {xs} {ws} stage={stage}", flush=True)
+        native.conv2d(out, xt, wt, bt, stride, dil, pad, memory_stage=stage)
+        return out
+
+    got, ref = conv(x, w, b, None).double(), conv(x, w, b, 2).double()
+    terms = conv(x.abs(), w.abs(), None, 2).double()
+    ulp = {"float32": 2.0 ** -22, "float16": 2.0 ** -10, "bfloat16": 2.0 ** -7}[dtype_name]
+    tol = ulp * ref.abs() + 2.0 ** -24 + 8 * k ** 0.5 * 2.0 ** -24 * terms
+    assert ((got - ref).abs() <= tol).all(), f"max err/tol {((got - ref).abs() / tol).max():.3g}"
+    flat = x.view(-1)
+    flat[torch.randint(0, flat.numel(), (7,), generator=gen, device=device)] = float("inf")
+    got, ref = conv(x, w, b, None), conv(x, w, b, 2)
+    assert torch.equal(torch.isfinite(got), torch.isfinite(ref)) and not torch.isfinite(ref).all()
