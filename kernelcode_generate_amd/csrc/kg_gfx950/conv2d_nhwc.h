@@ -45,8 +45,10 @@ struct Geometry {
   uint32_t row_h, row_w, img;   // bytes between output rows, output pixels, images
   uint32_t x_bytes;             // the copy's size
   uint32_t w_pitch;             // bytes per packed filter row
-  int bias_kind;  // 0 none, 1 fp32, 2 same dtype
+  int bias_kind;  // 0 none, 1 fp32, 2 same dtype; +2: one value per pixel instead of per filter
   int kcs;        // split-K: slices per split; 0 = all of them
+  int out_pitch;  // elements between filter rows of an image's output (Ho Wo)
+  int piece;      // output pixels per store: 8, 4 or 1 (rows start and end on multiples of it)
   FastDiv div_p, div_wo, div_spr, div_hpr, div_taps_w, div_pieces, div_hp, div_cpx, div_wrow, div_cp;
 };
 
@@ -415,11 +417,10 @@ __global__ __launch_bounds__(convn::kThreads, 2) void conv2d_nhwc_kernel(
   for (int j = 0; j < NB; ++j) {
     const int fr = wn * (BN / 2) + 16 * j + l16;
     const int f = f0 + fr;
-    float bv = 0.f;
-    if (!split && s.bias_kind != 0) {
-      const int fc = min(f, s.f - 1);
-      bv = s.bias_kind == 1 ? static_cast<const float*>(bias)[fc] : E::to_float(static_cast<const T*>(bias)[fc]);
-    }
+    auto bias_at = [&](int b) {
+      return s.bias_kind & 1 ? static_cast<const float*>(bias)[b] : E::to_float(static_cast<const T*>(bias)[b]);
+    };
+    const float bv = !split && (s.bias_kind == 1 || s.bias_kind == 2) ? bias_at(min(f, s.f - 1)) : 0.f;
 #pragma unroll
     for (int i = 0; i < MA; ++i) {
       const int px = wm * (BM / 2) + 16 * i + 4 * lg;
@@ -427,15 +428,20 @@ __global__ __launch_bounds__(convn::kThreads, 2) void conv2d_nhwc_kernel(
       if constexpr (KA == 4) r = (acc[0][i][j] + acc[1][i][j]) + (acc[2][i][j] + acc[3][i][j]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) r[e] += bv;
+      if (!split && s.bias_kind > 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] += bias_at(min(j0 + px + e, s.NP - 1));
+      }
       if (V == 4 || split) {
         // fp32 outputs or partial sums: straight from the registers
         float* out = split ? partial : reinterpret_cast<float*>(y);
+        const long long pitch = split ? s.P : s.out_pitch;
         if (f < s.f) {
-          if ((s.P & 3) == 0) {
+          if (split ? (s.P & 3) == 0 : s.piece >= 4) {
             const int jv = j0 + px;
             if (jv < s.NP) {
               const uint32_t n = fdiv((uint32_t)jv, s.div_p);
-              *reinterpret_cast<f32x4*>(out + ((long long)n * s.f + f) * s.P + (jv - n * s.P)) = r;
+              *reinterpret_cast<f32x4*>(out + ((long long)n * s.f + f) * pitch + (jv - n * s.P)) = r;
             }
           } else {
 #pragma unroll
@@ -443,7 +449,7 @@ __global__ __launch_bounds__(convn::kThreads, 2) void conv2d_nhwc_kernel(
               const int jv = j0 + px + e;
               if (jv < s.NP) {
                 const uint32_t n = fdiv((uint32_t)jv, s.div_p);
-                out[((long long)n * s.f + f) * s.P + (jv - n * s.P)] = r[e];
+                out[((long long)n * s.f + f) * pitch + (jv - n * s.P)] = r[e];
               }
             }
           }
@@ -459,7 +465,7 @@ __global__ __launch_bounds__(convn::kThreads, 2) void conv2d_nhwc_kernel(
   }
   if (V == 8 && !split) {
     __syncthreads();
-    // rows of BM pixels, G per lane; pieces of G lie in one image when P is a multiple of G
+    // rows of BM pixels, G per lane
     auto store_rows = [&](auto g_tag) {
       constexpr int G = decltype(g_tag)::value;
       using Piece = typename std::conditional<G == 8, u32x4, typename std::conditional<G == 4, u32x2, uint16_t>::type>::type;
@@ -470,16 +476,16 @@ __global__ __launch_bounds__(convn::kThreads, 2) void conv2d_nhwc_kernel(
       if (j >= s.NP) return;
       const uint32_t n = fdiv((uint32_t)j, s.div_p);
       const uint32_t p = j - n * s.P;
-      uint16_t* out = reinterpret_cast<uint16_t*>(y) + (long long)n * s.f * s.P + p;
+      uint16_t* out = reinterpret_cast<uint16_t*>(y) + (long long)n * s.f * s.out_pitch + p;
 #pragma unroll 4
       for (int r = tid / kLanes; r < BN; r += kRows) {
         if (f0 + r >= s.f) break;
-        *reinterpret_cast<Piece*>(out + (long long)(f0 + r) * s.P) =
+        *reinterpret_cast<Piece*>(out + (long long)(f0 + r) * s.out_pitch) =
             *reinterpret_cast<const Piece*>(lds + r * (BM * 2) + ((px >> 3) ^ out_mask(r)) * 16 + (px & 7) * 2);
       }
     };
-    if ((s.P & 7) == 0) store_rows(Int<8>{});
-    else if ((s.P & 3) == 0) store_rows(Int<4>{});
+    if (s.piece == 8) store_rows(Int<8>{});
+    else if (s.piece == 4) store_rows(Int<4>{});
     else store_rows(Int<1>{});
   }
 }
@@ -505,6 +511,8 @@ inline convn::Geometry conv_nhwc_geometry(const ConvShape& s, int images, int es
   g.slices = g.halves ? (s.kh * g.taps_w * g.hpr + 1) / 2 : s.kh * g.taps_w * g.spr;
   g.P = s.ho * s.wo;
   g.NP = images * g.P;
+  g.out_pitch = g.P;
+  g.piece = g.P % 8 == 0 ? 8 : g.P % 4 == 0 ? 4 : 1;
   const uint32_t px = (uint32_t)(g.cp * es);
   const uint32_t row = (uint32_t)g.wp * px;
   g.off_kh = (uint32_t)s.dh * row;
@@ -632,6 +640,25 @@ inline long long conv_nhwc_mfma(const ConvShape& s, const ConvNhwcPlan& plan, bo
   return n;
 }
 
+// The GEMM launch: tiles of bm pixels x 64 filters on a ring of `ring` stages.
+template <typename Tag>
+void launch_nhwc_gemm(const char* xp, const char* wp, typename convg::IgElem<Tag>::T* y, const void* bias,
+                      const convn::Geometry& g, int bm, int ring, int splits, float* partial, hipStream_t stream) {
+  const int grid = ((g.NP + bm - 1) / bm) * ((g.f + 63) / 64);
+#define KG_NHWC_GEMM(BM, R, HALVES)                                                                                 \
+  hipLaunchKernelGGL((conv2d_nhwc_kernel<Tag, BM, 64, R, HALVES>), dim3(grid, splits), dim3(convn::kThreads), 0, stream, \
+                     xp, wp, y, bias, g, partial)
+#define KG_NHWC_GEMM_H(BM, R) \
+  if (g.halves) KG_NHWC_GEMM(BM, R, true); else KG_NHWC_GEMM(BM, R, false)
+  if (bm == 128) {
+    if (ring == 2) { KG_NHWC_GEMM_H(128, 2); } else { KG_NHWC_GEMM_H(128, 3); }
+  } else {
+    if (ring == 3) { KG_NHWC_GEMM_H(64, 3); } else { KG_NHWC_GEMM_H(64, 5); }
+  }
+#undef KG_NHWC_GEMM_H
+#undef KG_NHWC_GEMM
+}
+
 template <typename Tag>
 hipError_t launch_conv2d_nhwc(const void* x, const void* w, void* y, const void* bias, int bias_kind,
                               const ConvShape& s, const ConvNhwcPlan& plan, char* ws, hipStream_t stream) {
@@ -653,20 +680,7 @@ hipError_t launch_conv2d_nhwc(const void* x, const void* w, void* y, const void*
     hipLaunchKernelGGL((conv_pack_kernel<Tag>), dim3(x_blocks + w_blocks), dim3(convn::kThreads), 0, stream, xs,
                        static_cast<const T*>(w), reinterpret_cast<u32x4*>(xpk), reinterpret_cast<u32x4*>(wpk), g, x_blocks);
     if (plan.splits > 1) g.kcs = plan.kcs;
-    const int grid = ((g.NP + plan.bm - 1) / plan.bm) * ((s.f + 63) / 64);
-#define KG_CONV_NHWC(BM, BN, R)                                                                                       \
-  if (g.halves)                                                                                                        \
-    hipLaunchKernelGGL((conv2d_nhwc_kernel<Tag, BM, BN, R, true>), dim3(grid, plan.splits), dim3(convn::kThreads), 0, \
-                       stream, xpk, wpk, ys, bias, g, partial);                                                       \
-  else                                                                                                                 \
-    hipLaunchKernelGGL((conv2d_nhwc_kernel<Tag, BM, BN, R, false>), dim3(grid, plan.splits), dim3(convn::kThreads), 0, \
-                       stream, xpk, wpk, ys, bias, g, partial)
-    if (plan.bm == 128) {
-      if (plan.ring == 2) { KG_CONV_NHWC(128, 64, 2); } else { KG_CONV_NHWC(128, 64, 3); }
-    } else {
-      if (plan.ring == 3) { KG_CONV_NHWC(64, 64, 3); } else { KG_CONV_NHWC(64, 64, 5); }
-    }
-#undef KG_CONV_NHWC
+    launch_nhwc_gemm<Tag>(xpk, wpk, ys, bias, g, plan.bm, plan.ring, plan.splits, partial, stream);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (plan.splits > 1) {

@@ -11,6 +11,7 @@
 #include "conv2d_rowvec.h"
 #include "flash_attn_mfma.h"
 #include "gemm.h"
+#include "gemm_packed.h"
 #include "gemm_quad.h"
 
 #ifdef KG_INSTANTIATE
@@ -130,6 +131,13 @@ KG_IGEMM_INSTANCE(F16Tag, 4)
 #define KG_NHWC_INSTANCE(TAG)                                                                                     \
   KG_INSTANCE hipError_t launch_conv2d_nhwc<TAG>(const void*, const void*, void*, const void*, int, const ConvShape&, \
                                                  const ConvNhwcPlan&, char*, hipStream_t);
+#define KG_GEMM_PACKED_INSTANCE(TAG)                                                                              \
+  KG_INSTANCE hipError_t launch_gemm_packed<TAG>(const void*, const void*, void*, const void*, int, int, int, int, \
+                                                 long long, long long, long long, const GemmPackedPlan&, char*, hipStream_t);
+KG_GEMM_PACKED_INSTANCE(F32Tag)
+KG_GEMM_PACKED_INSTANCE(Bf16Tag)
+KG_GEMM_PACKED_INSTANCE(F16Tag)
+#undef KG_GEMM_PACKED_INSTANCE
 KG_NHWC_INSTANCE(F32Tag)
 KG_NHWC_INSTANCE(Bf16Tag)
 KG_NHWC_INSTANCE(F16Tag)

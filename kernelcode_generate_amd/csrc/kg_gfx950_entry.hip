@@ -21,6 +21,7 @@
 #include "kg_gfx950/flash_attn.h"
 #include "kg_gfx950/gemm.h"
 #include "kg_gfx950/gemm_f32.h"
+#include "kg_gfx950/gemm_packed.h"
 #include "kg_gfx950/conv2d_mfma.h"
 #include "kg_gfx950/conv2d_igemm.h"
 #include "kg_gfx950/conv2d_nhwc.h"
@@ -539,9 +540,23 @@ int matmul_impl(const KgArgSlot* args, unsigned long long n) {
                            rhs.stride[0] % 4 == 0 && out.stride[0] % 4 == 0 && lhs.stride[0] <= kMaxPipeLd &&
                            rhs.stride[0] <= kMaxPipeLd && aligned16(lhs.data) && aligned16(rhs.data) &&
                            aligned16(out.data) && (!bias.present || bias.stride[0] == 1) && gemm_f32_mfma_pays(M, N, K);
+  // Calls left to the SIMT kernel by their alignment, once their K loop is worth two launches.
+  const bool f32 = out.dtype == KG_DTYPE_F32;
+  const bool simt = f32 ? !f32_mfma_ok && (!gemm_f32_splitk_ok(out, lhs, rhs, M, N, K) ||
+                                           (bias.present && bias.stride[0] != 1))
+                        : !mfma_ok;
+  const GemmPackedPlan packed = simt && !staged && gemm_packed_pays(M, N, K, f32) && lhs.stride[1] == 1 &&
+                                        rhs.stride[1] == 1 && out.stride[1] == 1 &&
+                                        out.stride[0] <= 0x7fffffff && (!bias.present || bias.stride[0] == 1)
+                                    ? gemm_packed_plan(M, N, K, f32, kSplitMaxWorkspace)
+                                    : GemmPackedPlan{};
+  const bool packed_ok = packed.ok;
   if (g_cost) {
     long long mfma = 0, cyc = 64;
-    if (f32_mfma_ok)  // 4 waves x 2 x 2 blocks x 8 k-steps (32x32x2) per 16-deep slice of a 128 x 128 tile
+    if (packed_ok) {  // 16x16x32, fp32 16x16x4
+      mfma = gemm_packed_mfma(M, N, packed, f32);
+      cyc = f32 ? 32 : 16;
+    } else if (f32_mfma_ok)  // 4 waves x 2 x 2 blocks x 8 k-steps (32x32x2) per 16-deep slice of a 128 x 128 tile
       mfma = cdiv(M, gemmf::kTile) * cdiv(N, gemmf::kTile) * cdiv(K, gemmf::kBK) * 128;
     else if (out.dtype == KG_DTYPE_F32 && gemm_f32_splitk_ok(out, lhs, rhs, M, N, K) &&
              (!bias.present || bias.stride[0] == 1))  // 8 MFMAs (32x32x2) per 32 x 32 block and 16-deep slice
@@ -558,6 +573,23 @@ int matmul_impl(const KgArgSlot* args, unsigned long long n) {
                        M * N * es);
   }
   if (M == 0 || N == 0) return finish_launch("matmul(empty)");
+  // (while a graph records, the workspace may not be used: it may be replaced later)
+  if (packed_ok && !stream_capturing()) {
+    SplitLease lease = split_workspace(packed.bytes(), g_stream);
+    if (char* ws = static_cast<char*>(lease.ptr)) {
+      const int bias_kind = !bias.present ? 0 : (bias.dtype == KG_DTYPE_F32 ? 1 : 2);
+      const void* bp = bias.present ? bias.data : nullptr;
+#define KG_GEMM_PACKED(TAG)                                                                                          \
+  launch_gemm_packed<TAG>(lhs.data, rhs.data, out.data, bp, bias_kind, m, nn, k, lhs.stride[0], rhs.stride[0],       \
+                          out.stride[0], packed, ws, g_stream)
+      const hipError_t e = out.dtype == KG_DTYPE_F32    ? KG_GEMM_PACKED(F32Tag)
+                           : out.dtype == KG_DTYPE_BF16 ? KG_GEMM_PACKED(Bf16Tag)
+                                                        : KG_GEMM_PACKED(F16Tag);
+#undef KG_GEMM_PACKED
+      if (e != hipSuccess) return fail(kHipFailure, "matmul(packed): %s", hipGetErrorString(e));
+      return finish_launch("matmul(packed)");
+    }
+  }
 
   if (out.dtype == KG_DTYPE_F32) {
     if (f32_mfma_ok) return launch_gemm_f32_mfma(out, lhs, rhs, bias, m, nn, k, (int)stages_f32);

@@ -466,3 +466,89 @@ def test_memory_stage_depths_bit_identical(device, oracle_mod, shape):
     assert_h16_close(to_numpy(default)[:64], ref, what=f"{shape} rows 0:64")
     with pytest.raises(native.NativeLibraryError, match="memory_stage"):
         native.call_entry("kg_gfx950_matmul_entry", (default, a, b, None, 64, 64, 64, 5))
+
+
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float16", "float32"])
+@pytest.mark.parametrize(
+    "shape,bias_kind,strided",
+    [
+        ((65, 1001, 129), "same", False),  # one column past a tile, K one past a chunk
+        ((301, 1001, 97), "f32", True),  # odd row strides and bases
+        ((1, 2003, 333), "none", False),  # one row, K split
+        ((130, 1000, 1003), "same", False),  # lhs aligned, rhs and out not
+        ((520, 1015, 520), "f32", True),  # K % 8 = 7: whole 8-column store pieces
+        ((3000, 1001, 1501), "none", False),  # 128-column tiles
+        ((700, 20011, 900), "same", False),  # rows that do not fit the workspace at once
+        ((33, 1000, 7), "none", False),  # fewer columns than a 16-byte piece
+    ],
+    ids=["edges", "strided", "row", "n_odd", "pieces8", "tiles128", "passes", "n7"],
+)
+def test_unaligned_rows_on_matrix_cores(device, shape, bias_kind, strided, dtype_name):
+    """Matmuls whose rows are not 16-byte aligned are packed into the workspace and run on the
+    channel-last GEMM (the entry's cost record shows the route). Reference: torch float64 on
+    the same inputs. Tolerance: the output's own rounding (half a spacing: 2^-8, 2^-11 and
+    2^-24 of the value, f16 2^-25 below its normal range) plus 4 sqrt(K) 2^-24 (|A| |B|), the
+    probabilistic bound for a K-term fp32 sum in any order (Higham and Mary, SIAM J. Sci. Comput.
+    41 (2019)). The output is a window of a NaN-filled buffer that must stay NaN outside it."""
+
+    import torch
+
+    dt = getattr(torch, dtype_name)
+    m, k, n = shape
+    gen = torch.Generator(device=device).manual_seed(m + 3 * k + 5 * n)
+
+    def draw(rows, cols, extra):
+        wide = torch.randn(rows, cols + extra, generator=gen, device=device).to(dt)
+        return wide[:, 3 : 3 + cols] if extra else wide
+
+    a, b = draw(m, k, 9 if strided else 0), draw(k, n, 8 if strided else 0)
+    bias = None if bias_kind == "none" else torch.randn(n, generator=gen, device=device)
+    if bias_kind == "same":
+        bias = bias.to(dt)
+    big = torch.full((m + 2, n + (8 if n % 8 == 0 else 3)), float("nan"), dtype=dt, device=device)
+    out = big[:m, :n]
+    spec = [native.TensorSpec.of(t) if t is not None else None for t in (out, a, b, bias)]
+    model = native.cost("matmul", spec)
+    assert model["MFMA"] > 0 and model["MFMA_CYCLES"] == model["MFMA"] * (32 if dt == torch.float32 else 16)
+    print(f"[matmul] packed {dtype_name} M={m} K={k} N={n} lda={a.stride(0)} ldb={b.stride(0)} ldc={out.stride(0)}", flush=True)
+    native.matmul(out, a, b, bias)
+    ref = a.double() @ b.double()
+    if bias is not None:
+        ref = ref + bias.double()
+    terms = a.double().abs() @ b.double().abs()
+    unit = {"float32": 2.0 ** -24, "float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}[dtype_name]
+    # the sum's error moves the value that is then rounded: twice the unit covers the crossing
+    tol = 2 * unit * ref.abs() + 2.0 ** -24 + 4 * k ** 0.5 * 2.0 ** -24 * terms
+    err = (out.double() - ref).abs()
+    assert (err <= tol).all(), f"max err/tol {(err / tol).max():.3g}"
+    assert torch.isnan(big[m:]).all() and torch.isnan(big[:, n:]).all(), "store outside the output window"
+
+
+def test_unaligned_rows_under_capture(device):
+    """While a graph records, the packed form's workspace is not used: the call keeps the SIMT
+    kernel, and every replay gives its bits."""
+
+    import torch
+
+    a = torch.randn(70, 1001, device=device).half()
+    b = torch.randn(1001, 99, device=device).half()
+    out = torch.empty(70, 99, dtype=torch.float16, device=device)
+    stream = torch.cuda.Stream(device=device)
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.graph(graph, stream=stream):
+            native.set_launch_mode(False, stream.cuda_stream)
+            native.matmul(out, a, b, None)
+    finally:
+        native.set_launch_mode(True, None)
+    ref = a.double() @ b.double()
+    tol = 2.0 ** -10 * ref.abs() + 2.0 ** -24 + 4 * 1001 ** 0.5 * 2.0 ** -24 * (a.double().abs() @ b.double().abs())
+    eager = torch.empty_like(out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ((out.double() - ref).abs() <= tol).all()
+        native.matmul(eager, a, b, None)
+        assert ((eager.double() - ref).abs() <= tol).all()
