@@ -1,0 +1,297 @@
+// Attention of few queries against many keys (a decoding step): 16-bit Q/K/V/O [B,H,S,D],
+// queries in blocks of 16, D in {64, 128}, fp32 online softmax, no mask.
+//
+// Such a call reads K and V once and does little else, so what bounds it is how much of the
+// chip keeps loads in flight. fa_fwd_mfma_kernel gives a (b,h) one workgroup (B H = 128: half
+// the CUs, 3.4 TB/s) whose K/V tiles wait for each other at barriers; here a (b,h)'s keys are
+// split over workgroups until there are two per CU, and each wave walks its own steps of keys
+// with its own running max and sums, its next step's K and V (16 KiB) in flight in registers
+// during the current one: no LDS, no barrier until the end.
+//
+// A step is kNC chunks of 32 keys. S^T = K Q^T as in flash_attn_mfma.h (v_mfma_f32_16x16x32,
+// operand A 16 keys x 32 d straight from K's rows, operand B Q^T in registers): lane l holds
+// the scores of query l%16 against keys 16kb + 4(l/16) + 0..3. O^T += V^T P^T contracts a chunk
+// in the key order a lane row holds P in, so lane row r needs V of keys 4r + 0..3 and 16 + 4r +
+// 0..3: it loads those 8 rows, D/16 columns per lane (whole rows per 16 lanes), and
+// transposes them in registers; block c of O^T is then rows d = (D/16) x + c, x = 0..15.
+// The waves' and then the splits' results (m, l, O) are combined as the online softmax does.
+#pragma once
+
+#include "common.h"
+#include "flash_attn.h"
+#include "flash_attn_mfma.h"
+
+namespace kg_gfx950 {
+
+namespace fad {
+constexpr int kWaves = 4;
+constexpr int kThreads = 64 * kWaves;
+constexpr int kMaxQ = 16;
+template <int D>
+constexpr int step_keys() { return D == 128 ? 32 : 64; }  // 16 KiB of K and V
+// The lowest running max: a score of -inf (infinite inputs) has weight 0 beside finite ones,
+// also where a whole step has no other.
+constexpr float kMinMax = -3.0e38f;
+}  // namespace fad
+
+// splits == 1: O is written; else partial[(bh splits + split) s_q + q][D + 2] takes O (not
+// normalised), m (log2 units) and l.
+template <typename Tag, int D>
+__global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint16_t* __restrict__ Q,
+                                                                     const uint16_t* __restrict__ K,
+                                                                     const uint16_t* __restrict__ V,
+                                                                     uint16_t* __restrict__ O, int s_q, int s_kv,
+                                                                     float scale_log2, int splits, int split_keys,
+                                                                     float* __restrict__ partial) {
+  using namespace fad;
+  using H = Half16<Tag>;
+  constexpr int NDS = D / 32;            // 32-deep d steps of S^T
+  constexpr int NE = D / 16;             // V columns per lane: blocks of O^T
+  constexpr int kStep = step_keys<D>();
+  constexpr int NC = kStep / 32;         // 32-key chunks per step
+  using VRow = typename std::conditional<NE == 8, u32x4, u32x2>::type;
+  struct Buf {
+    u32x4 k[2 * NC][NDS];
+    VRow v[NC][8];
+  };
+  __shared__ float o_lds[kWaves][kMaxQ][D];
+  __shared__ float ml_lds[kWaves][kMaxQ][2];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lr = lane >> 4;
+  const int bh = blockIdx.x / splits, split = blockIdx.x - bh * splits;
+  const int q0 = blockIdx.y * kMaxQ, nq = min(s_q - q0, kMaxQ);  // this workgroup's queries
+  const int key_lo = split * split_keys, key_hi = min(s_kv, key_lo + split_keys);
+  const uint16_t* Kb = K + (long long)bh * s_kv * D;
+  const uint16_t* Vb = V + (long long)bh * s_kv * D;
+
+  u32x4 qf[NDS];
+#pragma unroll
+  for (int s = 0; s < NDS; ++s)
+    qf[s] = l16 < nq ? ld16(Q + ((long long)bh * s_q + q0 + l16) * D + 32 * s + 8 * lr) : u32x4{0, 0, 0, 0};
+
+  // keys past key_hi (the last step of a range): rows of zeros
+  auto load = [&](Buf& b, int key0, bool whole) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kb = 0; kb < 2 * NC; ++kb) {
+      const int key = key0 + 16 * kb + l16;
+      const uint16_t* row = Kb + (long long)key * D + 8 * lr;
+#pragma unroll
+      for (int s = 0; s < NDS; ++s) b.k[kb][s] = whole || key < key_hi ? ld16(row + 32 * s) : u32x4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const int key = key0 + 32 * c + 4 * lr + (r < 4 ? r : 12 + r);
+        b.v[c][r] = whole || key < key_hi ? *reinterpret_cast<const VRow*>(Vb + (long long)key * D + NE * l16) : VRow{};
+      }
+  };
+
+  f32x4 o[NE];
+#pragma unroll
+  for (int c = 0; c < NE; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 l_run = {0.f, 0.f, 0.f, 0.f};
+  float m_run = kMinMax;
+  const u32x4 ones = {H::kOnePair, H::kOnePair, H::kOnePair, H::kOnePair};
+
+  auto compute = [&](Buf& b, int key0, bool whole) __attribute__((always_inline)) {
+    f32x4 sc[2 * NC];
+#pragma unroll
+    for (int kb = 0; kb < 2 * NC; ++kb) {
+      sc[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < NDS; ++s) sc[kb] = H::mfma16(b.k[kb][s], qf[s], sc[kb]);
+    }
+    if (!whole) {
+#pragma unroll
+      for (int kb = 0; kb < 2 * NC; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (key0 + 16 * kb + 4 * lr + i >= key_hi) sc[kb][i] = -INFINITY;
+    }
+    float mx = sc[0][0];
+#pragma unroll
+    for (int x = 1; x < 8 * NC; ++x) mx = __builtin_elementwise_maximum(mx, (float)sc[x >> 2][x & 3]);
+    float mx2 = mx;
+    fa::rows4_combine<true>(mx, mx2);
+    const float m_new = __builtin_elementwise_maximum(m_run, mx * scale_log2);
+    if (__builtin_amdgcn_ballot_w64(m_new > m_run || m_new != m_new)) {
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int c = 0; c < NE; ++c) o[c] *= alpha;
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      u32x4 pp;  // keys 32c + 4 lr + 0..3, then + 16
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[2 * c + h][2 * q], scale_log2, -m_run));
+          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[2 * c + h][2 * q + 1], scale_log2, -m_run));
+          pp[2 * h + q] = H::pack2(p0, p1);
+        }
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {  // column e of each lane's 8 rows
+        u32x4 vt;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t x = b.v[c][2 * q][e >> 1], y = b.v[c][2 * q + 1][e >> 1];
+          vt[q] = (e & 1) ? hi_halves(x, y) : lo_halves(x, y);
+        }
+        o[e] = H::mfma16(vt, pp, o[e]);
+      }
+      l_run = H::mfma16(ones, pp, l_run);
+    }
+  };
+
+  // this wave's steps: key_lo + kStep (wave + 4 i); all but the range's last are whole
+  constexpr int kStride = kStep * kWaves;
+  int key = key_lo + kStep * wave;
+  Buf b0, b1;
+  if (key + kStep <= key_hi) {
+    load(b0, key, true);
+    for (;;) {
+      const bool more1 = key + kStride + kStep <= key_hi;
+      if (more1) load(b1, key + kStride, true);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(b0, key, true);
+      key += kStride;
+      if (!more1) break;
+      const bool more0 = key + kStride + kStep <= key_hi;
+      if (more0) load(b0, key + kStride, true);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(b1, key, true);
+      key += kStride;
+      if (!more0) break;
+    }
+  }
+  if (key < key_hi) {
+    load(b0, key, false);
+    compute(b0, key, false);
+  }
+
+  // ---- combine the waves ----
+  if (l16 < nq) {
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o_lds[wave][l16][NE * (4 * lr + i) + e] = o[e][i];
+    if (lr == 0) {
+      ml_lds[wave][l16][0] = m_run;
+      ml_lds[wave][l16][1] = l_run[0];
+    }
+  }
+  __syncthreads();
+  for (int x = tid; x < nq * (D / 2); x += kThreads) {
+    const int q = x / (D / 2), d = 2 * (x % (D / 2));
+    float m = ml_lds[0][q][0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) m = __builtin_elementwise_maximum(m, ml_lds[w][q][0]);
+    float l = 0.f, o0 = 0.f, o1 = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const float a = __builtin_amdgcn_exp2f(ml_lds[w][q][0] - m);
+      l += a * ml_lds[w][q][1];
+      o0 += a * o_lds[w][q][d];
+      o1 += a * o_lds[w][q][d + 1];
+    }
+    if (splits == 1) {
+      const float inv = 1.f / l;
+      *reinterpret_cast<uint32_t*>(O + ((long long)bh * s_q + q0 + q) * D + d) = H::pack2(o0 * inv, o1 * inv);
+    } else {
+      float* p = partial + ((long long)blockIdx.x * s_q + q0 + q) * (D + 2);
+      *reinterpret_cast<f32x2*>(p + d) = f32x2{o0, o1};
+      if (d == 0) *reinterpret_cast<f32x2*>(p + D) = f32x2{m, l};
+    }
+  }
+}
+
+// One wave per (b,h) and query: the splits' partials combined and normalised, D / 64 columns per lane.
+template <typename Tag, int D>
+__global__ __launch_bounds__(64) void fa_decode_combine_kernel(const float* __restrict__ partial,
+                                                               uint16_t* __restrict__ O, int s_q, int splits) {
+  const int lane = threadIdx.x;
+  const int bh = blockIdx.x / s_q, q = blockIdx.x - bh * s_q;
+  const float* p = partial + ((long long)bh * splits * s_q + q) * (D + 2);
+  const long long pitch = (long long)s_q * (D + 2);
+  float m = -INFINITY;
+  for (int s = lane; s < splits; s += 64) m = fmaxf(m, p[s * pitch + D]);
+  m = wave_max(m);
+  float l = 0.f, o[D / 64];
+#pragma unroll
+  for (int e = 0; e < D / 64; ++e) o[e] = 0.f;
+#pragma unroll 8
+  for (int s = 0; s < splits; ++s) {
+    const float a = __builtin_amdgcn_exp2f(p[s * pitch + D] - m);
+    l += a * p[s * pitch + D + 1];
+#pragma unroll
+    for (int e = 0; e < D / 64; ++e) o[e] += a * p[s * pitch + lane + 64 * e];
+  }
+  const float inv = 1.f / l;
+#pragma unroll
+  for (int e = 0; e < D / 64; ++e)
+    O[((long long)bh * s_q + q) * D + lane + 64 * e] = (uint16_t)(Half16<Tag>::pack2(o[e] * inv, 0.f) & 0xffffu);
+}
+
+// The calls it takes: up to 16 queries always; more, in blocks of 16 that each read the keys
+// again, while the blocks are few beside the 512 workgroups that fill the chip and the keys many
+// (us, this kernel / fa_fwd_mfma_kernel, bf16, B H x S_q x S_kv x D: 128x1x4096x128 44 / 81,
+// 8x1x16384x128 17 / 298, 8x64x16384x128 30 / 299, 8x128x1024x128 14.6 / 19.2, 128x17x2048x128 (256
+// blocks) 43 / 43, 32x128x4096x128 (256 blocks) 47 / 64, 256x17x1000x128 (512 blocks) 38 / 32).
+inline int fa_decode_blocks(const FaShape& s) { return (s.s_q + fad::kMaxQ - 1) / fad::kMaxQ; }
+inline bool fa_decode_supported(const FaShape& s) {
+  const long long blocks = (long long)s.bh * fa_decode_blocks(s);
+  const bool pays = s.s_q <= fad::kMaxQ ||
+                    (s.s_kv >= 1024 && (blocks <= 128 || (blocks <= 256 && s.s_q >= 64 && s.s_kv >= 2048)));
+  return s.s_q >= 1 && s.s_kv >= 1 && !s.causal && (s.d == 64 || s.d == 128) && s.scale > 0.f && s.bh >= 1 &&
+         s.bh <= (1 << 20) && pays;
+}
+
+// Splits of a call's keys (ranges of whole steps): two workgroups per CU of the MI355X (256),
+// each wave with at least two steps. splits == 1 needs no workspace.
+struct FaDecodePlan {
+  int splits, split_keys;
+  size_t bytes;  // of partials
+};
+inline FaDecodePlan fa_decode_plan(const FaShape& s, bool may_split) {
+  const int step = s.d == 128 ? fad::step_keys<128>() : fad::step_keys<64>();
+  const long long rounds = ((long long)s.s_kv + step * fad::kWaves - 1) / (step * fad::kWaves);  // steps per wave in all
+  long long splits = std::min<long long>(512 / ((long long)s.bh * fa_decode_blocks(s)), rounds / 2);
+  if (splits < 2 || !may_split) return FaDecodePlan{1, s.s_kv, 0};
+  const long long per = (rounds + splits - 1) / splits;
+  splits = (rounds + per - 1) / per;
+  return FaDecodePlan{(int)splits, (int)(per * step * fad::kWaves),
+                      splits > 1 ? (size_t)s.bh * splits * s.s_q * (s.d + 2) * sizeof(float) : 0};
+}
+// MFMA instructions: per step 2 S^T blocks x D/32 and D/16 + 1 for O^T and the row sums per chunk.
+inline long long fa_decode_mfma(const FaShape& s) {
+  const int step = s.d == 128 ? fad::step_keys<128>() : fad::step_keys<64>();
+  return (long long)s.bh * fa_decode_blocks(s) * ((s.s_kv + step - 1) / step) * (step / 32) * (s.d / 16 + s.d / 16 + 1);
+}
+
+template <typename Tag, int D>
+hipError_t launch_fa_decode_d(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* o, const FaShape& s,
+                              const FaDecodePlan& plan, float* partial, hipStream_t stream) {
+  hipLaunchKernelGGL((fa_decode_kernel<Tag, D>), dim3(s.bh * plan.splits, fa_decode_blocks(s)),
+                     dim3(fad::kThreads), 0, stream, q, k, v, o,
+                     s.s_q, s.s_kv, s.scale * 1.4426950408889634f, plan.splits, plan.split_keys, partial);
+  if (plan.splits > 1)
+    hipLaunchKernelGGL((fa_decode_combine_kernel<Tag, D>), dim3(s.bh * s.s_q), dim3(64), 0, stream, partial, o, s.s_q,
+                       plan.splits);
+  return hipGetLastError();
+}
+
+template <typename Tag>
+hipError_t launch_fa_decode(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* o, const FaShape& s,
+                            const FaDecodePlan& plan, float* partial, hipStream_t stream) {
+  if (s.d == 128) return launch_fa_decode_d<Tag, 128>(q, k, v, o, s, plan, partial, stream);
+  return launch_fa_decode_d<Tag, 64>(q, k, v, o, s, plan, partial, stream);
+}
+
+}  // namespace kg_gfx950

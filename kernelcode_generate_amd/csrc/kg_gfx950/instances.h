@@ -9,6 +9,7 @@
 #include "conv2d_mfma.h"
 #include "conv2d_nhwc.h"
 #include "conv2d_rowvec.h"
+#include "flash_attn_decode.h"
 #include "flash_attn_mfma.h"
 #include "gemm.h"
 #include "gemm_packed.h"
@@ -85,6 +86,15 @@ KG_FA_INSTANCE(F16Tag, 2)
 KG_FA_INSTANCE(F16Tag, 3)
 KG_FA_INSTANCE(F16Tag, 4)
 #undef KG_FA_INSTANCE
+#endif
+
+#if !defined(KG_INSTANTIATE) || defined(KG_INSTANTIATE_FA_DECODE)
+#define KG_FA_DECODE_INSTANCE(TAG)                                                                                   \
+  KG_INSTANCE hipError_t launch_fa_decode<TAG>(const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*,        \
+                                               const FaShape&, const FaDecodePlan&, float*, hipStream_t);
+KG_FA_DECODE_INSTANCE(Bf16Tag)
+KG_FA_DECODE_INSTANCE(F16Tag)
+#undef KG_FA_DECODE_INSTANCE
 #endif
 
 #if !defined(KG_INSTANTIATE) || defined(KG_INSTANTIATE_CONV_ROWVEC)

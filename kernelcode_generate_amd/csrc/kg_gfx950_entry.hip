@@ -27,6 +27,7 @@
 #include "kg_gfx950/conv2d_nhwc.h"
 #include "kg_gfx950/conv2d_rowvec.h"
 #include "kg_gfx950/flash_attn_mfma.h"
+#include "kg_gfx950/flash_attn_decode.h"
 #include "kg_gfx950/flash_attn_f32.h"
 #include "kg_gfx950/instances.h"  // the heavy kernel families are compiled in their own translation units
 
@@ -903,12 +904,19 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
   if (g_cost == nullptr && out.numel() == 0) return finish_launch("flash_attention(empty)");
   if (s.d > 512) return fail(kUnsupported, "flash_attention: head dim %d > 512", s.d);
   if (s.causal && s.s_kv != s.s_q) return fail(kUnsupported, "flash_attention: causal mask needs S_q == S_kv");
+  // few queries: keys split over workgroups (a call that sets a ring depth takes the kernel with
+  // the ring)
+  const bool decode = (out.dtype == KG_DTYPE_BF16 || out.dtype == KG_DTYPE_F16) && !staged && out.numel() > 0 &&
+                      fa_decode_supported(s) && aligned16(q.data) && aligned16(k.data) && aligned16(v.data) &&
+                      aligned16(out.data);
   if (g_cost) {
     const long long B_H = (long long)s.bh, D = s.d;
     // products Q.K^T and P.V that the mask keeps: causal row i sees keys 0..i
     const long long pairs = s.causal ? (long long)s.s_q * (s.s_q + 1) / 2 : (long long)s.s_q * s.s_kv;
     long long mfma = 0;
-    if ((out.dtype == KG_DTYPE_BF16 || out.dtype == KG_DTYPE_F16) && fa_mfma_supported(s) && out.numel() > 0) {
+    if (decode) {
+      mfma = fa_decode_mfma(s);
+    } else if ((out.dtype == KG_DTYPE_BF16 || out.dtype == KG_DTYPE_F16) && fa_mfma_supported(s) && out.numel() > 0) {
       // per workgroup: waves x key tiles x (D/4 16x16x32 MFMAs for S^T + D/4 for PV + 4 row sums)
       const int waves = fa_mfma_waves(s);
       const int bm = 32 * waves;
@@ -943,6 +951,25 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
                        (q.numel() + k.numel() + v.numel()) * es, out.numel() * es);
   }
 
+  if (decode) {
+    // one range per (b,h) where there is no workspace, or while a graph records (it may be
+    // replaced later)
+    FaDecodePlan plan = fa_decode_plan(s, true);
+    SplitLease lease;
+    if (plan.splits > 1) {
+      if (!stream_capturing()) lease = split_workspace(plan.bytes, g_stream);
+      if (lease.ptr == nullptr) plan = fa_decode_plan(s, false);
+    }
+    float* partial = static_cast<float*>(lease.ptr);
+    const uint16_t *qp = static_cast<const uint16_t*>(q.data), *kp = static_cast<const uint16_t*>(k.data),
+                   *vp = static_cast<const uint16_t*>(v.data);
+    uint16_t* op = static_cast<uint16_t*>(out.data);
+    const hipError_t e = out.dtype == KG_DTYPE_BF16
+                             ? launch_fa_decode<Bf16Tag>(qp, kp, vp, op, s, plan, partial, g_stream)
+                             : launch_fa_decode<F16Tag>(qp, kp, vp, op, s, plan, partial, g_stream);
+    if (e != hipSuccess) return fail(kHipFailure, "flash_attention(decode): %s", hipGetErrorString(e));
+    return finish_launch("flash_attention(decode)");
+  }
   if ((out.dtype == KG_DTYPE_BF16 || out.dtype == KG_DTYPE_F16) && fa_mfma_supported(s) && aligned16(q.data) &&
       aligned16(k.data) && aligned16(v.data) && aligned16(out.data)) {
     hipError_t e = out.dtype == KG_DTYPE_BF16

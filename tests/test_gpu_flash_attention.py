@@ -307,3 +307,82 @@ def test_rejects_bad_args(device):
         native.flash_attention(o, q, q, q, 0, 4)
     with pytest.raises(native.NativeLibraryError):
         native.call_entry("kg_gfx950_flash_attention_entry", (o, q, q, q, 4, 4, 1.0, 2))
+
+
+DECODE = [
+    # (b, h, s_q, s_kv, d): one step of keys, a step's edges, ranges that end mid-step, splits
+    (1, 2, 1, 1, 128), (2, 1, 3, 31, 64), (1, 3, 16, 33, 128), (1, 2, 7, 64, 64), (2, 3, 1, 257, 128),
+    (1, 5, 2, 4097, 128), (3, 2, 16, 2049, 64), (4, 32, 1, 1000, 128),
+    (1, 3, 17, 1030, 128), (1, 2, 300, 1025, 64),  # blocks of 16 queries, the last one partial
+]
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("b,h,s_q,s_kv,d", DECODE)
+def test_few_queries(device, b, h, s_q, s_kv, d, dtype):
+    """Few queries take the kernel that splits the keys over workgroups (the entry's cost record
+    shows the route). Reference: the softmax formula in float64 on the rounded inputs; bar:
+    gpu_util.attention_h16_tolerance. The first 40 keys of a head with more are then made to
+    score -inf for every query (whole steps without a finite score): they must weigh nothing."""
+
+    import torch
+
+    from tests.gpu_util import attention_h16_tolerance
+
+    tdt = getattr(torch, dtype)
+    rng = np.random.default_rng(s_q + s_kv + d)
+    q, qn = round_to(rng.standard_normal((b, h, s_q, d), dtype=np.float32), tdt)
+    (k, kn), (v, vn) = (round_to(rng.standard_normal((b, h, s_kv, d), dtype=np.float32), tdt) for _ in range(2))
+    scale = 1.0 / np.sqrt(d)
+    steps, chunks = (-(-s_kv // 32), 1) if d == 128 else (-(-s_kv // 64), 2)
+    specs = [native.TensorSpec(x, dtype) for x in (q.shape, q.shape, k.shape, k.shape)]
+    assert native.cost("flash_attention", [*specs, 64, 64, scale, 0])["MFMA"] == \
+        b * h * -(-s_q // 16) * steps * chunks * (d // 8 + 1)
+
+    def check(qn, kn, what):
+        out = torch.full(q.shape, float("nan"), dtype=tdt, device=device)
+        print(f"[fa] few queries {what} {(b, h, s_q, s_kv, d)} {dtype}", flush=True)
+        native.flash_attention(out, torch.from_numpy(qn).to(tdt).to(device), torch.from_numpy(kn).to(tdt).to(device),
+                               v.to(device), 64, 64, scale, False)
+        live = np.isfinite(kn).all(axis=(0, 1, 3))
+        s = qn.astype(np.float64) @ kn[:, :, live].astype(np.float64).swapaxes(-1, -2) * scale
+        w = np.exp(s - s.max(-1, keepdims=True))
+        ref = (w / w.sum(-1, keepdims=True)) @ vn[:, :, live].astype(np.float64)
+        tol = attention_h16_tolerance(qn, kn[:, :, live], vn[:, :, live], scale, False, dtype)
+        assert_within(to_numpy(out), ref, tol, what=what)
+
+    check(qn, kn, "normal")
+    if s_kv > 60:
+        dead = kn.copy()
+        dead[:, :, :40] = -np.inf
+        check(np.abs(qn) + np.float32(0.125), dead, "dead keys")
+
+
+def test_few_queries_under_capture(device):
+    """While a graph records, the keys of a (b,h) are not split (no workspace); every replay
+    gives the softmax formula's result."""
+
+    import torch
+
+    q = torch.randn(1, 2, 1, 128, device=device).bfloat16()
+    k, v = (torch.randn(1, 2, 3000, 128, device=device).bfloat16() for _ in range(2))
+    out = torch.empty_like(q)
+    stream = torch.cuda.Stream(device=device)
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.graph(graph, stream=stream):
+            native.set_launch_mode(False, stream.cuda_stream)
+            native.flash_attention(out, q, k, v, 64, 64, 0.088, False)
+    finally:
+        native.set_launch_mode(True, None)
+    qd, kd, vd = (t.double()[0] for t in (q, k, v))
+    ref = torch.stack([torch.softmax(0.088 * (qd[i] @ kd[i].t().contiguous()), -1) @ vd[i] for i in range(2)])
+    eager = torch.empty_like(out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        native.flash_attention(eager, q, k, v, 64, 64, 0.088, False)
+        torch.cuda.synchronize()
+        for got in (out, eager):
+            assert_h16_close(to_numpy(got[0]), ref.cpu().numpy(), what="replay")
