@@ -18,6 +18,7 @@
 #pragma once
 
 #include "common.h"
+#include "conv2d_igemm.h"
 #include "flash_attn.h"
 #include "flash_attn_mfma.h"
 
@@ -36,12 +37,13 @@ constexpr float kMinMax = -3.0e38f;
 
 // splits == 1: O is written; else partial[(bh splits + split) s_q + q][D + 2] takes O (not
 // normalised), m (log2 units) and l.
-template <typename Tag, int D>
+// kAny: head dims d < D (multiples of 8, rows padded with zeros in registers) and causal calls.
+template <typename Tag, int D, bool kAny>
 __global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint16_t* __restrict__ Q,
                                                                      const uint16_t* __restrict__ K,
                                                                      const uint16_t* __restrict__ V,
-                                                                     uint16_t* __restrict__ O, int s_q, int s_kv,
-                                                                     float scale_log2, int splits, int split_keys,
+                                                                     uint16_t* __restrict__ O, int s_q, int s_kv, int d_any,
+                                                                     int causal, float scale_log2, int splits, int split_keys,
                                                                      float* __restrict__ partial) {
   using namespace fad;
   using H = Half16<Tag>;
@@ -63,30 +65,39 @@ __global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint1
   const int l16 = lane & 15, lr = lane >> 4;
   const int bh = blockIdx.x / splits, split = blockIdx.x - bh * splits;
   const int q0 = blockIdx.y * kMaxQ, nq = min(s_q - q0, kMaxQ);  // this workgroup's queries
-  const int key_lo = split * split_keys, key_hi = min(s_kv, key_lo + split_keys);
-  const uint16_t* Kb = K + (long long)bh * s_kv * D;
-  const uint16_t* Vb = V + (long long)bh * s_kv * D;
+  const int d_row = kAny ? d_any : D;
+  const bool diagonal = kAny && causal != 0;
+  const int key_lo = split * split_keys;
+  const int key_hi = min(diagonal ? min(s_kv, q0 + nq) : s_kv, key_lo + split_keys);
+  const uint16_t* Kb = K + (long long)bh * s_kv * d_row;
+  const uint16_t* Vb = V + (long long)bh * s_kv * d_row;
 
   u32x4 qf[NDS];
 #pragma unroll
   for (int s = 0; s < NDS; ++s)
-    qf[s] = l16 < nq ? ld16(Q + ((long long)bh * s_q + q0 + l16) * D + 32 * s + 8 * lr) : u32x4{0, 0, 0, 0};
+    qf[s] = l16 < nq && (!kAny || 32 * s + 8 * lr < d_row)
+                ? ld16(Q + ((long long)bh * s_q + q0 + l16) * d_row + 32 * s + 8 * lr)
+                : u32x4{0, 0, 0, 0};
 
   // keys past key_hi (the last step of a range): rows of zeros
   auto load = [&](Buf& b, int key0, bool whole) __attribute__((always_inline)) {
 #pragma unroll
     for (int kb = 0; kb < 2 * NC; ++kb) {
       const int key = key0 + 16 * kb + l16;
-      const uint16_t* row = Kb + (long long)key * D + 8 * lr;
+      const uint16_t* row = Kb + (long long)key * d_row + 8 * lr;
 #pragma unroll
-      for (int s = 0; s < NDS; ++s) b.k[kb][s] = whole || key < key_hi ? ld16(row + 32 * s) : u32x4{0, 0, 0, 0};
+      for (int s = 0; s < NDS; ++s)
+        b.k[kb][s] = (whole || key < key_hi) && (!kAny || 32 * s + 8 * lr < d_row) ? ld16(row + 32 * s)
+                                                                                   : u32x4{0, 0, 0, 0};
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int r = 0; r < 8; ++r) {
         const int key = key0 + 32 * c + 4 * lr + (r < 4 ? r : 12 + r);
-        b.v[c][r] = whole || key < key_hi ? *reinterpret_cast<const VRow*>(Vb + (long long)key * D + NE * l16) : VRow{};
+        b.v[c][r] = (whole || key < key_hi) && (!kAny || NE * l16 < d_row)
+                        ? *reinterpret_cast<const VRow*>(Vb + (long long)key * d_row + NE * l16)
+                        : VRow{};
       }
   };
 
@@ -105,12 +116,13 @@ __global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint1
 #pragma unroll
       for (int s = 0; s < NDS; ++s) sc[kb] = H::mfma16(b.k[kb][s], qf[s], sc[kb]);
     }
-    if (!whole) {
+    if (!whole || (diagonal && key0 + kStep - 1 > q0)) {
+      const int last = diagonal ? min(key_hi - 1, q0 + l16) : key_hi - 1;  // this query's last key
 #pragma unroll
       for (int kb = 0; kb < 2 * NC; ++kb)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (key0 + 16 * kb + 4 * lr + i >= key_hi) sc[kb][i] = -INFINITY;
+          if (key0 + 16 * kb + 4 * lr + i > last) sc[kb][i] = -INFINITY;
     }
     float mx = sc[0][0];
 #pragma unroll
@@ -190,6 +202,7 @@ __global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint1
   __syncthreads();
   for (int x = tid; x < nq * (D / 2); x += kThreads) {
     const int q = x / (D / 2), d = 2 * (x % (D / 2));
+    if (kAny && d >= d_row) continue;
     float m = ml_lds[0][q][0];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) m = __builtin_elementwise_maximum(m, ml_lds[w][q][0]);
@@ -203,7 +216,7 @@ __global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint1
     }
     if (splits == 1) {
       const float inv = 1.f / l;
-      *reinterpret_cast<uint32_t*>(O + ((long long)bh * s_q + q0 + q) * D + d) = H::pack2(o0 * inv, o1 * inv);
+      *reinterpret_cast<uint32_t*>(O + ((long long)bh * s_q + q0 + q) * d_row + d) = H::pack2(o0 * inv, o1 * inv);
     } else {
       float* p = partial + ((long long)blockIdx.x * s_q + q0 + q) * (D + 2);
       *reinterpret_cast<f32x2*>(p + d) = f32x2{o0, o1};
@@ -215,7 +228,8 @@ __global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint1
 // One wave per (b,h) and query: the splits' partials combined and normalised, D / 64 columns per lane.
 template <typename Tag, int D>
 __global__ __launch_bounds__(64) void fa_decode_combine_kernel(const float* __restrict__ partial,
-                                                               uint16_t* __restrict__ O, int s_q, int splits) {
+                                                               typename convg::IgElem<Tag>::T* __restrict__ O, int s_q,
+                                                               int d_row, int splits) {
   const int lane = threadIdx.x;
   const int bh = blockIdx.x / s_q, q = blockIdx.x - bh * s_q;
   const float* p = partial + ((long long)bh * splits * s_q + q) * (D + 2);
@@ -235,8 +249,176 @@ __global__ __launch_bounds__(64) void fa_decode_combine_kernel(const float* __re
   }
   const float inv = 1.f / l;
 #pragma unroll
-  for (int e = 0; e < D / 64; ++e)
-    O[((long long)bh * s_q + q) * D + lane + 64 * e] = (uint16_t)(Half16<Tag>::pack2(o[e] * inv, 0.f) & 0xffffu);
+  for (int e = 0; e < D / 64; ++e) {
+    const int d = lane + 64 * e;
+    if (d >= d_row) continue;
+    auto* out = O + ((long long)bh * s_q + q) * d_row + d;
+    if constexpr (convg::IgElem<Tag>::kPerChunk == 8) *out = (uint16_t)(Half16<Tag>::pack2(o[e] * inv, 0.f) & 0xffffu);
+    else *out = o[e] * inv;
+  }
+}
+
+// fp32 form (v_mfma_f32_16x16x4_f32, one k per lane), any head dim d <= 16 NE that is a multiple
+// of 4, causal or not: a step is 16 keys; S^T takes 16 d in four MFMAs from 16-byte pieces of K's
+// rows (element j of every lane's piece), O^T takes the keys 4(l/16) + i of a step in MFMA i
+// against V[key][16 e + l%16], which needs no transpose. fa_fwd_simt_kernel, one workgroup per
+// query, read every key row once per query and lane: 16x389x389x80 took 133 us.
+template <int NE>
+__global__ __launch_bounds__(fad::kThreads, 2) void fa_split_f32_kernel(const float* __restrict__ Q,
+                                                                        const float* __restrict__ K,
+                                                                        const float* __restrict__ V,
+                                                                        float* __restrict__ O, int s_q, int s_kv, int d_row,
+                                                                        int causal, float scale_log2, int splits,
+                                                                        int split_keys, float* __restrict__ partial) {
+  using namespace fad;
+  constexpr int D = NE <= 4 ? 64 : 128;  // columns of a partial row
+  constexpr int kStep = 16;
+  struct Buf {
+    f32x4 k[NE];
+    float v[4][NE];
+  };
+  __shared__ float o_lds[kWaves][kMaxQ][16 * NE + 1];
+  __shared__ float ml_lds[kWaves][kMaxQ][2];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lr = lane >> 4;
+  const int bh = blockIdx.x / splits, split = blockIdx.x - bh * splits;
+  const int q0 = blockIdx.y * kMaxQ, nq = min(s_q - q0, kMaxQ);
+  const int key_lo = split * split_keys;
+  const int key_hi = min(causal ? min(s_kv, q0 + nq) : s_kv, key_lo + split_keys);
+  const float* Kb = K + (long long)bh * s_kv * d_row;
+  const float* Vb = V + (long long)bh * s_kv * d_row;
+  const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+
+  f32x4 qf[NE];
+#pragma unroll
+  for (int s = 0; s < NE; ++s)
+    qf[s] = l16 < nq && 16 * s + 4 * lr < d_row
+                ? *reinterpret_cast<const f32x4*>(Q + ((long long)bh * s_q + q0 + l16) * d_row + 16 * s + 4 * lr)
+                : zero4;
+
+  auto load = [&](Buf& b, int key0) __attribute__((always_inline)) {
+    const int kk = key0 + l16;
+#pragma unroll
+    for (int s = 0; s < NE; ++s)
+      b.k[s] = kk < key_hi && 16 * s + 4 * lr < d_row
+                   ? *reinterpret_cast<const f32x4*>(Kb + (long long)kk * d_row + 16 * s + 4 * lr)
+                   : zero4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int key = key0 + 4 * lr + i;
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+        b.v[i][e] = key < key_hi && 16 * e + l16 < d_row ? Vb[(long long)key * d_row + 16 * e + l16] : 0.f;
+    }
+  };
+
+  f32x4 o[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) o[e] = zero4;
+  float l_run = 0.f;  // this lane's keys' share of the row sum
+  float m_run = kMinMax;
+  auto compute = [&](Buf& b, int key0) __attribute__((always_inline)) {
+    // two accumulators: half as long a chain of dependent MFMAs
+    f32x4 sc = zero4, sd = zero4;
+#pragma unroll
+    for (int s = 0; s < NE; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        f32x4& acc = j & 1 ? sd : sc;
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32((float)b.k[s][j], (float)qf[s][j], acc, 0, 0, 0);
+      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sc[i] += sd[i];
+    const int last = causal ? min(key_hi - 1, q0 + l16) : key_hi - 1;  // this query's last key
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (key0 + 4 * lr + i > last) sc[i] = -INFINITY;
+    float mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum((float)sc[0], (float)sc[1]),
+                                             __builtin_elementwise_maximum((float)sc[2], (float)sc[3]));
+    float mx2 = mx;
+    fa::rows4_combine<true>(mx, mx2);
+    const float m_new = __builtin_elementwise_maximum(m_run, mx * scale_log2);
+    if (__builtin_amdgcn_ballot_w64(m_new > m_run || m_new != m_new)) {
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) o[e] *= alpha;
+    }
+    float p[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf((float)sc[i], scale_log2, -m_run));
+      l_run += p[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < NE; ++e) o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.v[i][e], p[i], o[e], 0, 0, 0);
+  };
+
+  constexpr int kStride = kStep * kWaves;
+  Buf b0, b1;
+  int key = key_lo + kStep * wave;
+  if (key < key_hi) {
+    load(b0, key);
+    for (;;) {
+      const bool more1 = key + kStride < key_hi;
+      if (more1) load(b1, key + kStride);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(b0, key);
+      key += kStride;
+      if (!more1) break;
+      const bool more0 = key + kStride < key_hi;
+      if (more0) load(b0, key + kStride);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(b1, key);
+      key += kStride;
+      if (!more0) break;
+    }
+  }
+
+  // the four lane rows' row sums, then the waves
+  float l2 = l_run;
+  fa::rows4_combine<false>(l_run, l2);
+  if (l16 < nq) {
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o_lds[wave][l16][16 * e + 4 * lr + i] = o[e][i];
+    if (lr == 0) {
+      ml_lds[wave][l16][0] = m_run;
+      ml_lds[wave][l16][1] = l_run;
+    }
+  }
+  __syncthreads();
+  for (int x = tid; x < nq * 16 * NE; x += kThreads) {
+    const int q = x / (16 * NE), d = x % (16 * NE);
+    if (d >= d_row) continue;
+    float m = ml_lds[0][q][0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) m = __builtin_elementwise_maximum(m, ml_lds[w][q][0]);
+    float l = 0.f, ov = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const float a = __builtin_amdgcn_exp2f(ml_lds[w][q][0] - m);
+      l += a * ml_lds[w][q][1];
+      ov += a * o_lds[w][q][d];
+    }
+    if (splits == 1) {
+      O[((long long)bh * s_q + q0 + q) * d_row + d] = ov / l;
+    } else {
+      float* p = partial + ((long long)blockIdx.x * s_q + q0 + q) * (D + 2);
+      p[d] = ov;
+      if (d == 0) {
+        p[D] = m;
+        p[D + 1] = l;
+      }
+    }
+  }
 }
 
 // The calls it takes: up to 16 queries always; more, in blocks of 16 that each read the keys
@@ -252,6 +434,20 @@ inline bool fa_decode_supported(const FaShape& s) {
   return s.s_q >= 1 && s.s_kv >= 1 && !s.causal && (s.d == 64 || s.d == 128) && s.scale > 0.f && s.bh >= 1 &&
          s.bh <= (1 << 20) && pays;
 }
+// Head dims the tiled kernels do not have, which otherwise run one workgroup per query (16-bit:
+// multiples of 8 from 24, fp32: of 4; causal or not), any call (us, this kernel /
+// fa_fwd_simt_kernel: 16x389x389x80 fp32 26 / 139, bf16 9.5 / 104; 128x512x512x96 causal bf16 48 /
+// 775). Below 24 the padding to 64 is most of the work. And fp32 with D = 64 or 128, causal or not, of up
+// to 16 queries or 512 blocks of them, where fa_fwd_f32_mfma_kernel's blocks of 128 queries leave
+// CUs idle (8x1x8192x128 23 / 1179; 16x512x512x64 22 / 47; 24x64x64x64 10.5 / 9.5, x128 10.7 / 13.5;
+// 256x64x64x64, 1024 blocks, 11.9 / 9.4; 32x1024x1024x64, 2048 blocks, 151 / 95).
+inline bool fa_split_supported(const FaShape& s, bool f32) {
+  if (!(s.s_q >= 1 && s.s_kv >= 1 && s.scale > 0.f && s.bh >= 1 && s.bh <= (1 << 20) && fa_decode_blocks(s) <= 65535))
+    return false;
+  if (s.d != 64 && s.d != 128) return s.d >= 24 && s.d <= 128 && s.d % (f32 ? 4 : 8) == 0;
+  if (f32) return s.s_q <= fad::kMaxQ || (long long)s.bh * fa_decode_blocks(s) <= 512;
+  return fa_decode_supported(s);
+}
 
 // Splits of a call's keys (ranges of whole steps): two workgroups per CU of the MI355X (256),
 // each wave with at least two steps. splits == 1 needs no workspace.
@@ -259,39 +455,77 @@ struct FaDecodePlan {
   int splits, split_keys;
   size_t bytes;  // of partials
 };
-inline FaDecodePlan fa_decode_plan(const FaShape& s, bool may_split) {
-  const int step = s.d == 128 ? fad::step_keys<128>() : fad::step_keys<64>();
+inline FaDecodePlan fa_decode_plan(const FaShape& s, bool f32, bool may_split) {
+  const int step = f32 ? 16 : s.d > 64 ? fad::step_keys<128>() : fad::step_keys<64>();
+  const int cols = s.d > 64 ? 128 : 64;
   const long long rounds = ((long long)s.s_kv + step * fad::kWaves - 1) / (step * fad::kWaves);  // steps per wave in all
   long long splits = std::min<long long>(512 / ((long long)s.bh * fa_decode_blocks(s)), rounds / 2);
   if (splits < 2 || !may_split) return FaDecodePlan{1, s.s_kv, 0};
   const long long per = (rounds + splits - 1) / splits;
   splits = (rounds + per - 1) / per;
   return FaDecodePlan{(int)splits, (int)(per * step * fad::kWaves),
-                      splits > 1 ? (size_t)s.bh * splits * s.s_q * (s.d + 2) * sizeof(float) : 0};
+                      splits > 1 ? (size_t)s.bh * splits * s.s_q * (cols + 2) * sizeof(float) : 0};
 }
-// MFMA instructions: per step 2 S^T blocks x D/32 and D/16 + 1 for O^T and the row sums per chunk.
-inline long long fa_decode_mfma(const FaShape& s) {
-  const int step = s.d == 128 ? fad::step_keys<128>() : fad::step_keys<64>();
-  return (long long)s.bh * fa_decode_blocks(s) * ((s.s_kv + step - 1) / step) * (step / 32) * (s.d / 16 + s.d / 16 + 1);
+// MFMA instructions: per step and block of queries 2 S^T blocks x D/32 and D/16 + 1 for O^T and the
+// row sums per 32 keys; fp32 4 for S^T and 4 for O^T per 16 d and 16 keys. Causal blocks stop at
+// their last query's step.
+inline long long fa_decode_mfma(const FaShape& s, bool f32, const FaDecodePlan& plan) {
+  const int step = f32 ? 16 : s.d > 64 ? fad::step_keys<128>() : fad::step_keys<64>();
+  const int D = s.d > 64 ? 128 : 64, NE = s.d <= 64 ? 4 : s.d <= 96 ? 6 : 8;
+  long long steps = 0;
+  for (int b = 0; b < fa_decode_blocks(s); ++b) {
+    const int end = s.causal ? std::min(s.s_kv, std::min((b + 1) * fad::kMaxQ, s.s_q)) : s.s_kv;
+    for (long long lo = 0; lo < end; lo += plan.split_keys)
+      steps += (std::min<long long>(plan.split_keys, end - lo) + step - 1) / step;
+  }
+  return s.bh * steps * (f32 ? 8 * NE : (step / 32) * (D / 16 + D / 16 + 1));
 }
 
-template <typename Tag, int D>
+template <typename Tag, int D, bool kAny>
 hipError_t launch_fa_decode_d(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* o, const FaShape& s,
                               const FaDecodePlan& plan, float* partial, hipStream_t stream) {
-  hipLaunchKernelGGL((fa_decode_kernel<Tag, D>), dim3(s.bh * plan.splits, fa_decode_blocks(s)),
-                     dim3(fad::kThreads), 0, stream, q, k, v, o,
-                     s.s_q, s.s_kv, s.scale * 1.4426950408889634f, plan.splits, plan.split_keys, partial);
+  hipLaunchKernelGGL((fa_decode_kernel<Tag, D, kAny>), dim3(s.bh * plan.splits, fa_decode_blocks(s)),
+                     dim3(fad::kThreads), 0, stream, q, k, v, o, s.s_q, s.s_kv, s.d, s.causal,
+                     s.scale * 1.4426950408889634f, plan.splits, plan.split_keys, partial);
   if (plan.splits > 1)
     hipLaunchKernelGGL((fa_decode_combine_kernel<Tag, D>), dim3(s.bh * s.s_q), dim3(64), 0, stream, partial, o, s.s_q,
-                       plan.splits);
+                       s.d, plan.splits);
   return hipGetLastError();
 }
 
 template <typename Tag>
 hipError_t launch_fa_decode(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* o, const FaShape& s,
                             const FaDecodePlan& plan, float* partial, hipStream_t stream) {
-  if (s.d == 128) return launch_fa_decode_d<Tag, 128>(q, k, v, o, s, plan, partial, stream);
-  return launch_fa_decode_d<Tag, 64>(q, k, v, o, s, plan, partial, stream);
+  if (s.causal || (s.d != 64 && s.d != 128)) {
+    if (s.d > 64) return launch_fa_decode_d<Tag, 128, true>(q, k, v, o, s, plan, partial, stream);
+    return launch_fa_decode_d<Tag, 64, true>(q, k, v, o, s, plan, partial, stream);
+  }
+  if (s.d == 128) return launch_fa_decode_d<Tag, 128, false>(q, k, v, o, s, plan, partial, stream);
+  return launch_fa_decode_d<Tag, 64, false>(q, k, v, o, s, plan, partial, stream);
+}
+
+template <int NE>
+void launch_fa_split_f32_ne(const float* q, const float* k, const float* v, float* o, const FaShape& s,
+                            const FaDecodePlan& plan, float* partial, hipStream_t stream) {
+  hipLaunchKernelGGL((fa_split_f32_kernel<NE>), dim3(s.bh * plan.splits, fa_decode_blocks(s)), dim3(fad::kThreads), 0,
+                     stream, q, k, v, o, s.s_q, s.s_kv, s.d, s.causal, s.scale * 1.4426950408889634f, plan.splits,
+                     plan.split_keys, partial);
+}
+template <typename Tag>
+hipError_t launch_fa_split_f32(const float* q, const float* k, const float* v, float* o, const FaShape& s,
+                               const FaDecodePlan& plan, float* partial, hipStream_t stream) {
+  if (s.d <= 64) launch_fa_split_f32_ne<4>(q, k, v, o, s, plan, partial, stream);
+  else if (s.d <= 96) launch_fa_split_f32_ne<6>(q, k, v, o, s, plan, partial, stream);
+  else launch_fa_split_f32_ne<8>(q, k, v, o, s, plan, partial, stream);
+  if (plan.splits > 1) {
+    if (s.d <= 64)
+      hipLaunchKernelGGL((fa_decode_combine_kernel<Tag, 64>), dim3(s.bh * s.s_q), dim3(64), 0, stream, partial, o, s.s_q,
+                         s.d, plan.splits);
+    else
+      hipLaunchKernelGGL((fa_decode_combine_kernel<Tag, 128>), dim3(s.bh * s.s_q), dim3(64), 0, stream, partial, o,
+                         s.s_q, s.d, plan.splits);
+  }
+  return hipGetLastError();
 }
 
 }  // namespace kg_gfx950

@@ -95,6 +95,8 @@ KG_FA_INSTANCE(F16Tag, 4)
 KG_FA_DECODE_INSTANCE(Bf16Tag)
 KG_FA_DECODE_INSTANCE(F16Tag)
 #undef KG_FA_DECODE_INSTANCE
+KG_INSTANCE hipError_t launch_fa_split_f32<F32Tag>(const float*, const float*, const float*, float*, const FaShape&,
+                                                     const FaDecodePlan&, float*, hipStream_t);
 #endif
 
 #if !defined(KG_INSTANTIATE) || defined(KG_INSTANTIATE_CONV_ROWVEC)

@@ -904,10 +904,10 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
   if (g_cost == nullptr && out.numel() == 0) return finish_launch("flash_attention(empty)");
   if (s.d > 512) return fail(kUnsupported, "flash_attention: head dim %d > 512", s.d);
   if (s.causal && s.s_kv != s.s_q) return fail(kUnsupported, "flash_attention: causal mask needs S_q == S_kv");
-  // few queries: keys split over workgroups (a call that sets a ring depth takes the kernel with
+  // few queries, or a head dim of its own: keys split over workgroups (a call that sets a ring depth takes the kernel with
   // the ring)
-  const bool decode = (out.dtype == KG_DTYPE_BF16 || out.dtype == KG_DTYPE_F16) && !staged && out.numel() > 0 &&
-                      fa_decode_supported(s) && aligned16(q.data) && aligned16(k.data) && aligned16(v.data) &&
+  const bool f32 = out.dtype == KG_DTYPE_F32;
+  const bool decode = !staged && out.numel() > 0 && fa_split_supported(s, f32) && aligned16(q.data) && aligned16(k.data) && aligned16(v.data) &&
                       aligned16(out.data);
   if (g_cost) {
     const long long B_H = (long long)s.bh, D = s.d;
@@ -915,7 +915,7 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
     const long long pairs = s.causal ? (long long)s.s_q * (s.s_q + 1) / 2 : (long long)s.s_q * s.s_kv;
     long long mfma = 0;
     if (decode) {
-      mfma = fa_decode_mfma(s);
+      mfma = fa_decode_mfma(s, f32, fa_decode_plan(s, f32, true));
     } else if ((out.dtype == KG_DTYPE_BF16 || out.dtype == KG_DTYPE_F16) && fa_mfma_supported(s) && out.numel() > 0) {
       // per workgroup: waves x key tiles x (D/4 16x16x32 MFMAs for S^T + D/4 for PV + 4 row sums)
       const int waves = fa_mfma_waves(s);
@@ -928,7 +928,7 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
       }
       mfma = B_H * tiles * waves * (s.d / 2 + 4);
     }
-    if (out.dtype == KG_DTYPE_F32 && fa_f32_mfma_supported(s) && out.numel() > 0) {
+    if (!decode && f32 && fa_f32_mfma_supported(s) && out.numel() > 0) {
       // per workgroup and key tile: D MFMAs (32x32x2: D/2 for S^T, D/2 for PV) per wave that
       // has a query and (causal) a visible key in the tile
       const int nqb = (s.s_q + faf::kBM - 1) / faf::kBM;
@@ -947,20 +947,27 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
       mfma = B_H * waves_tiles * s.d;
     }
     const long long es = esize(out.dtype);
-    return record_cost(2 * B_H * pairs * D, mfma, out.dtype == KG_DTYPE_F32 ? 64 : 16,
+    return record_cost(2 * B_H * pairs * D, mfma, !f32 ? 16 : decode ? 32 : 64,
                        (q.numel() + k.numel() + v.numel()) * es, out.numel() * es);
   }
 
   if (decode) {
     // one range per (b,h) where there is no workspace, or while a graph records (it may be
     // replaced later)
-    FaDecodePlan plan = fa_decode_plan(s, true);
+    FaDecodePlan plan = fa_decode_plan(s, f32, true);
     SplitLease lease;
     if (plan.splits > 1) {
       if (!stream_capturing()) lease = split_workspace(plan.bytes, g_stream);
-      if (lease.ptr == nullptr) plan = fa_decode_plan(s, false);
+      if (lease.ptr == nullptr) plan = fa_decode_plan(s, f32, false);
     }
     float* partial = static_cast<float*>(lease.ptr);
+    if (f32) {
+      const hipError_t e = launch_fa_split_f32<F32Tag>(static_cast<const float*>(q.data), static_cast<const float*>(k.data),
+                                                       static_cast<const float*>(v.data), static_cast<float*>(out.data), s,
+                                                       plan, partial, g_stream);
+      if (e != hipSuccess) return fail(kHipFailure, "flash_attention(split f32): %s", hipGetErrorString(e));
+      return finish_launch("flash_attention(split f32)");
+    }
     const uint16_t *qp = static_cast<const uint16_t*>(q.data), *kp = static_cast<const uint16_t*>(k.data),
                    *vp = static_cast<const uint16_t*>(v.data);
     uint16_t* op = static_cast<uint16_t*>(out.data);

@@ -5,9 +5,10 @@ counter run can be laid beside the model:
 
 Every case makes one library MFMA kernel dispatch, in the order printed, followed (for the
 conv cases whose grid is small enough to split K) by a split-K reduction kernel that issues
-no MFMA; inputs are generated on the host and copied, and the only other
+no MFMA (and, where operands are packed first or keys are split, their packing or combine
+kernel); inputs are generated on the host and copied, and the only other
 dispatches are the HIP runtime's own copy kernels (named __amd_rocclr_*) that some
-host-to-device copies use, so leaving out those and the *_splitk_reduce_kernel dispatches,
+host-to-device copies use, so leaving out those and the *_splitk_reduce_kernel, *_pack_kernel and *_combine_kernel dispatches,
 library dispatch i of the counter run is case i. Cases cover every kernel choice the model distinguishes: the
 pipelined MFMA GEMM with 256- and 128-row tiles and with ragged edges, the fp32 MFMA GEMM
 aligned and ragged, the fp32 split-K GEMM, the SIMT GEMM, the MFMA conv with four and with two live waves and a
@@ -60,6 +61,9 @@ CASES = (
     ("fa_f16_causal_1x2x1000x64", "flash_attention", "float16", ((1, 2, 1000, 64),) * 4, (128, 64, 0.125, 1)),
     ("fa_bf16_2x3x130x128", "flash_attention", "bfloat16", ((2, 3, 130, 128),) * 4, (128, 64, 0.088388, 0)),
     ("fa_f32_causal_1x2x700x128", "flash_attention", "float32", ((1, 2, 700, 128),) * 4, (64, 64, 0.088388, 1)),
+    ("fa_f32_causal_1x40x250x64", "flash_attention", "float32", ((1, 40, 250, 64),) * 4, (64, 64, 0.125, 1)),
+    ("fa_bf16_2x3x100x80", "flash_attention", "bfloat16", ((2, 3, 100, 80),) * 4, (64, 64, 0.125, 1)),
+    ("gemm_f16_packed_301x999x777", "matmul", "float16", ((301, 999), (301, 777), (777, 999)), ()),
     ("fa_f32_2x1x130x64", "flash_attention", "float32", ((2, 1, 130, 64),) * 4, (64, 64, 0.125, 0)),
 )
 

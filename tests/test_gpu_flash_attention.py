@@ -386,3 +386,49 @@ def test_few_queries_under_capture(device):
         torch.cuda.synchronize()
         for got in (out, eager):
             assert_h16_close(to_numpy(got[0]), ref.cpu().numpy(), what="replay")
+
+
+ANY_DIM = [
+    # (b, h, s_q, s_kv, d, causal): dims with and without whole 16-column blocks, blocks of 16 queries
+    # with a partial last one, split keys (few heads), one step, more steps than waves
+    (1, 2, 70, 70, 24, True), (2, 1, 33, 130, 40, False), (1, 3, 257, 257, 48, True), (1, 1, 16, 1000, 72, False),
+    (1, 2, 300, 300, 80, True), (2, 2, 100, 65, 96, False), (1, 1, 1, 33, 120, False), (1, 1, 700, 700, 104, True),
+]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("b,h,s_q,s_kv,d,causal", ANY_DIM + [(1, 5, 77, 77, 64, True), (1, 2, 16, 500, 128, False)])
+def test_any_head_dim(device, b, h, s_q, s_kv, d, causal, dtype):
+    """Head dims without a tiled kernel (and small fp32 calls with D = 64 and 128) take the
+    split-key kernels. Reference: the softmax formula in float64; bars: gpu_util's, plus for
+    fp32 the float64 reference's distance to the bar's own. The inputs sit in buffers whose other
+    elements are NaN, so a read outside a row's columns shows."""
+
+    import torch
+
+    from tests.gpu_util import attention_h16_tolerance
+
+    tdt = getattr(torch, dtype)
+    rng = np.random.default_rng(s_q + s_kv + d)
+    arrays, tensors = [], []
+    for s in (s_q, s_kv, s_kv):
+        t, a = round_to(rng.standard_normal((b, h, s, d), dtype=np.float32), tdt)
+        guard = torch.full((t.numel() + 512,), float("nan"), dtype=tdt, device=device)
+        guard[256 : 256 + t.numel()] = t.flatten().to(device)
+        arrays.append(a)
+        tensors.append(guard[256 : 256 + t.numel()].view(b, h, s, d))
+    scale = 1.0 / np.sqrt(d)
+    guard = torch.full((b * h * s_q * d + 512,), float("nan"), dtype=tdt, device=device)
+    out = guard[256:-256].view(b, h, s_q, d)
+    print(f"[fa] any dim {(b, h, s_q, s_kv, d)} causal={causal} {dtype}", flush=True)
+    native.flash_attention(out, *tensors, 64, 64, scale, causal)
+    qn, kn, vn = (a.astype(np.float64) for a in arrays)
+    s = qn @ kn.swapaxes(-1, -2) * scale
+    if causal:
+        s = np.where(np.tril(np.ones((s_q, s_kv), bool)), s, -np.inf)
+    w = np.exp(s - s.max(-1, keepdims=True))
+    ref = (w / w.sum(-1, keepdims=True)) @ vn
+    tol = attention_f32_tolerance(*arrays, scale, causal) if dtype == "float32" else \
+        attention_h16_tolerance(*arrays, scale, causal, dtype)
+    assert_within(to_numpy(out), ref, tol, what=f"{(b, h, s_q, s_kv, d)} {causal} {dtype}")
+    assert torch.isnan(guard[:256]).all() and torch.isnan(guard[-256:]).all(), "store outside the output"
