@@ -12,6 +12,7 @@
 #include "flash_attn_decode.h"
 #include "flash_attn_mfma.h"
 #include "gemm.h"
+#include "gemm_mid.h"
 #include "gemm_packed.h"
 #include "gemm_quad.h"
 
@@ -40,6 +41,20 @@ KG_GEMM_PIPE_INSTANCES(F16Tag, 256, false)
 KG_GEMM_PIPE_INSTANCES(F16Tag, 256, true)
 #undef KG_GEMM_PIPE_INSTANCES
 #undef KG_GEMM_PIPE_INSTANCE
+#endif
+
+#if !defined(KG_INSTANTIATE) || defined(KG_INSTANTIATE_GEMM_MID)
+#define KG_GEMM_MID_INSTANCE(TAG, ST, RAG)                                                                             \
+  KG_INSTANCE hipError_t launch_gemm_mid<TAG, ST, RAG>(const uint16_t*, const uint16_t*, uint16_t*, const void*, int, int, \
+                                                       int, int, long long, long long, long long, hipStream_t);
+#define KG_GEMM_MID_INSTANCES(TAG)                                      \
+  KG_GEMM_MID_INSTANCE(TAG, 2, false) KG_GEMM_MID_INSTANCE(TAG, 2, true) \
+  KG_GEMM_MID_INSTANCE(TAG, 3, false) KG_GEMM_MID_INSTANCE(TAG, 3, true) \
+  KG_GEMM_MID_INSTANCE(TAG, 4, false) KG_GEMM_MID_INSTANCE(TAG, 4, true)
+KG_GEMM_MID_INSTANCES(Bf16Tag)
+KG_GEMM_MID_INSTANCES(F16Tag)
+#undef KG_GEMM_MID_INSTANCES
+#undef KG_GEMM_MID_INSTANCE
 #endif
 
 #if !defined(KG_INSTANTIATE) || defined(KG_INSTANTIATE_GEMM_QUAD)

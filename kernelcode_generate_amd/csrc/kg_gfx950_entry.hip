@@ -21,6 +21,7 @@
 #include "kg_gfx950/flash_attn.h"
 #include "kg_gfx950/gemm.h"
 #include "kg_gfx950/gemm_f32.h"
+#include "kg_gfx950/gemm_mid.h"
 #include "kg_gfx950/gemm_packed.h"
 #include "kg_gfx950/conv2d_mfma.h"
 #include "kg_gfx950/conv2d_igemm.h"
@@ -370,9 +371,29 @@ SplitLease split_workspace(size_t bytes, hipStream_t stream) {
   return lease;
 }
 
+// 128 x 128 tiles (gemm_mid_kernel) where they make one round on the chip: half the work per
+// workgroup of 128 x 256 ones, which then leave CUs idle. Not where so few tiles have so long a K
+// that splitting K wins. us, this kernel / 128 x 256 tiles, split over K where they were: 2048^3
+// 18.5 / 25.3, 2048x2048x512 8.3 / 10.4, 1536x1536x8192 50 / 65, 2304x2304x2048 (324 tiles) 28 / 26,
+// 5887x1792x3712 (644) 118 / 103; few tiles, split: 1024^3 10.2 / 16.6, 16x4096x1024 11.2 / 10.8,
+// 512x1024x2048 15.2 / 21.6, 371x256x1472 15.6 / 13.4, 64x4096x2048 18.3 / 14.7, 1280x1280x8192 49 / 58,
+// 2745x512x7552 (44 wide tiles) 54 / 48, 1024x1024x4096 26 / 24, 200x8192x4096 31 / 29. Up to K = 512 also grids of up to two rounds
+// (2176x2048: 9.8 / 10.5).
+bool gemm_mid_pays(long long M, long long N, long long K) {
+  if (pipe_tile_m(M, N) != 128) return false;
+  const long long mid = cdiv(M, gemmm::kT) * cdiv(N, gemmm::kT), wide = cdiv(M, 128) * cdiv(N, gemmp::kBN);
+  if (mid > kNumCUs) return K <= 512 && mid <= 2 * kNumCUs;
+  if (wide > kSplitMaxTiles || K <= 1024) return true;
+  if (K <= 2048) return wide >= 12 && std::min(M, N) >= 192;
+  return wide > 48 && std::min(M, N) >= 512;
+}
+// Its ring: four stages of a 64-deep slice, or two and two workgroups per CU where the K loop is
+// short beside its fill (2048x2048x1024: 11.3 us with two stages, 12.0 with four; x2048: 24.2, 18.5).
+int gemm_mid_stages(long long K) { return K <= 1024 ? 2 : 4; }
+
 template <typename Tag>
 int launch_gemm_mfma(const Mem& out, const Mem& lhs, const Mem& rhs, const Mem& bias, int M, int N, int K,
-                     int stages) {
+                     int stages, bool staged) {
   const uint16_t* A = static_cast<const uint16_t*>(lhs.data);
   const uint16_t* B = static_cast<const uint16_t*>(rhs.data);
   uint16_t* C = static_cast<uint16_t*>(out.data);
@@ -385,6 +406,17 @@ int launch_gemm_mfma(const Mem& out, const Mem& lhs, const Mem& rhs, const Mem& 
   const int grid = (int)(cdiv(M, tm) * cdiv(N, gemmp::kBN));
   long long chunk = K;
   int splits = pipe_splits(M, N, K, &chunk);
+  if (gemm_mid_pays(M, N, K)) {
+    const int depth = staged ? stages : gemm_mid_stages(K);
+    const bool edges = M % gemmm::kT || N % gemmm::kT || K % gemmm::kBK;
+#define KG_GEMM_MID(ST)                                                                                                   \
+  (edges ? launch_gemm_mid<Tag, ST, true>(A, B, C, bp, bias_kind, M, N, K, lda, ldb, ldc, g_stream)                       \
+         : launch_gemm_mid<Tag, ST, false>(A, B, C, bp, bias_kind, M, N, K, lda, ldb, ldc, g_stream))
+    const hipError_t e = depth == 2 ? KG_GEMM_MID(2) : depth == 3 ? KG_GEMM_MID(3) : KG_GEMM_MID(4);
+#undef KG_GEMM_MID
+    if (e != hipSuccess) return fail(kHipFailure, "matmul(mfma-mid): %s", hipGetErrorString(e));
+    return finish_launch("matmul(mfma-mid)");
+  }
   float* partial = nullptr;
   SplitLease lease;  // held until both kernels of a split call are enqueued (this function's return)
   if (splits > 1) {
@@ -567,6 +599,8 @@ int matmul_impl(const KgArgSlot* args, unsigned long long n) {
       // whole 256 x 256 tiles 4 waves x 64; ragged edges are covered by whole tiles and slices
       const long long tm = pipe_tile_m(M, N);
       mfma = cdiv(M, tm) * cdiv(N, gemmp::kBN) * cdiv(K, gemmp::kBK) * tm;
+      if (gemm_mid_pays(M, N, K))  // 4 waves x 16 per 32-deep step of a 128 x 128 tile, two steps a slice
+        mfma = cdiv(M, gemmm::kT) * cdiv(N, gemmm::kT) * cdiv(K, gemmm::kBK) * 128;
       cyc = 16;
     }
     const long long es = esize(out.dtype);
@@ -605,11 +639,11 @@ int matmul_impl(const KgArgSlot* args, unsigned long long n) {
     return fail(kUnsupported, "matmul: memory_stage sets the LDS ring depth of the MFMA kernels; this call takes the "
                               "SIMT kernel, which stages nothing through an LDS ring");
   if (out.dtype == KG_DTYPE_BF16) {
-    if (mfma_ok) return launch_gemm_mfma<Bf16Tag>(out, lhs, rhs, bias, m, nn, k, (int)stages);
+    if (mfma_ok) return launch_gemm_mfma<Bf16Tag>(out, lhs, rhs, bias, m, nn, k, (int)stages, staged);
     if (bias.present && bias.dtype == KG_DTYPE_F32) return launch_gemm_simt<__bf16, float>(out, lhs, rhs, bias, m, nn, k);
     return launch_gemm_simt<__bf16, __bf16>(out, lhs, rhs, bias, m, nn, k);
   }
-  if (mfma_ok) return launch_gemm_mfma<F16Tag>(out, lhs, rhs, bias, m, nn, k, (int)stages);
+  if (mfma_ok) return launch_gemm_mfma<F16Tag>(out, lhs, rhs, bias, m, nn, k, (int)stages, staged);
   if (bias.present && bias.dtype == KG_DTYPE_F32) return launch_gemm_simt<_Float16, float>(out, lhs, rhs, bias, m, nn, k);
   return launch_gemm_simt<_Float16, _Float16>(out, lhs, rhs, bias, m, nn, k);
 }

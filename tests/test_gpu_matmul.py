@@ -552,3 +552,48 @@ def test_unaligned_rows_under_capture(device):
         assert ((out.double() - ref).abs() <= tol).all()
         native.matmul(eager, a, b, None)
         assert ((eager.double() - ref).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
+@pytest.mark.parametrize(
+    "shape,bias_kind",
+    [
+        ((2048, 2048, 2048), "f32"),  # 256 whole tiles, four stages
+        ((1536, 1024, 1408), "same"),  # whole tiles, 22 slices
+        ((1024, 8, 1024), "none"),  # a fraction of one slice
+        ((1000, 72, 1000), "f32"),  # one slice and 8 k, ragged rows and columns
+        ((129, 512, 136), "same"),  # one row and 8 columns past a tile
+        ((700, 1208, 2056), "none"),  # ragged everywhere, 19 slices
+        ((2176, 192, 2048), "same"),  # K <= 512, 272 tiles
+    ],
+    ids=["2048", "whole22", "k8", "k72", "edges", "ragged", "shortk"],
+)
+def test_128_tiles_match_wide_tiles(device, shape, bias_kind, dtype_name):
+    """128 x 128 tiles against the 128 x 256-tile kernel on the same columns: every output block is
+    the same sequence of 32-deep MFMAs, so the bits agree at every ring depth. The wide tiles
+    come from a call whose output is wide enough for them (rhs repeated to the right until
+    there are more than two rounds of tiles; K not split then); the first columns are compared. The
+    output is a window of a NaN-filled buffer."""
+
+    import torch
+
+    dt = getattr(torch, dtype_name)
+    m, k, n = shape
+    gen = torch.Generator(device=device).manual_seed(m + k + n)
+    a = (torch.randn(m, k, generator=gen, device=device) * 0.1).to(dt)
+    b = (torch.randn(k, n, generator=gen, device=device) * 0.1).to(dt)
+    bias = None if bias_kind == "none" else torch.randn(n, generator=gen, device=device)
+    if bias_kind == "same":
+        bias = bias.to(dt)
+    reps = 1
+    while -(-m // 128) * -(-n * reps // 256) <= 770:
+        reps += 1
+    wide = torch.empty(m, n * reps, dtype=dt, device=device)
+    print(f"[matmul] 128-tiles {shape} {dtype_name} reps={reps}", flush=True)
+    native.matmul(wide, a, b.repeat(1, reps), None if bias is None else bias.repeat(reps))
+    for stages in (None, 2, 3, 4):
+        big = torch.full((m + 2, n + 8), float("nan"), dtype=dt, device=device)
+        args = (big[:m, :n], a, b, bias) + (() if stages is None else (64, 64, 64, stages))
+        native.call_entry("kg_gfx950_matmul_entry", args)
+        assert torch.equal(big[:m, :n], wide[:, :n]), f"stages={stages}"
+        assert torch.isnan(big[m:]).all() and torch.isnan(big[:, n:]).all(), "store outside the output window"
