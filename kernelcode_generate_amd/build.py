@@ -46,7 +46,7 @@ def include_flags() -> list[str]:
 
 SOURCES = ("kg_gfx950_entry.hip", "kg_gfx950_gemm.hip", "kg_gfx950_gemm_quad.hip", "kg_gfx950_gemm_mid.hip", "kg_gfx950_fa.hip",
            "kg_gfx950_fa_persist.hip", "kg_gfx950_fa_decode.hip", "kg_gfx950_conv_rowvec.hip", "kg_gfx950_conv_igemm.hip",
-           "kg_gfx950_conv_nhwc.hip")
+           "kg_gfx950_conv_nhwc.hip", "kg_gfx950_gemm_skinny.hip")
 
 
 def build_library(output: Path = OUTPUT, extra_flags: tuple[str, ...] = (), verbose: bool = False) -> Path:

@@ -15,6 +15,7 @@
 #include "gemm_mid.h"
 #include "gemm_packed.h"
 #include "gemm_quad.h"
+#include "gemm_skinny.h"
 
 #ifdef KG_INSTANTIATE
 #define KG_INSTANCE template
@@ -55,6 +56,16 @@ KG_GEMM_MID_INSTANCES(Bf16Tag)
 KG_GEMM_MID_INSTANCES(F16Tag)
 #undef KG_GEMM_MID_INSTANCES
 #undef KG_GEMM_MID_INSTANCE
+#endif
+
+#if !defined(KG_INSTANTIATE) || defined(KG_INSTANTIATE_GEMM_SKINNY)
+#define KG_GEMM_SKINNY_INSTANCE(TAG)                                                                                     \
+  KG_INSTANCE hipError_t launch_gemm_skinny<TAG>(const void*, const void*, void*, const void*, int, int, int, int,       \
+                                                 long long, long long, long long, hipStream_t);
+KG_GEMM_SKINNY_INSTANCE(F32Tag)
+KG_GEMM_SKINNY_INSTANCE(Bf16Tag)
+KG_GEMM_SKINNY_INSTANCE(F16Tag)
+#undef KG_GEMM_SKINNY_INSTANCE
 #endif
 
 #if !defined(KG_INSTANTIATE) || defined(KG_INSTANTIATE_GEMM_QUAD)

@@ -23,6 +23,7 @@
 #include "kg_gfx950/gemm_f32.h"
 #include "kg_gfx950/gemm_mid.h"
 #include "kg_gfx950/gemm_packed.h"
+#include "kg_gfx950/gemm_skinny.h"
 #include "kg_gfx950/conv2d_mfma.h"
 #include "kg_gfx950/conv2d_igemm.h"
 #include "kg_gfx950/conv2d_nhwc.h"
@@ -526,6 +527,30 @@ int launch_gemm_f32_splitk(const Mem& out, const Mem& lhs, const Mem& rhs, const
   return finish_launch("matmul(f32-splitk)");
 }
 
+// Few rows: one round of workgroups that each read their columns of rhs once, against kernels that
+// copy tiles through LDS and split K over two launches. mfma: the call meets the alignment of
+// those (splitk: of the fp32 kernel of 32 x 32 blocks); otherwise the packed form or the SIMT
+// kernel would take it. us, this kernel / the other:
+// - 16-bit, aligned: one round, 16x4096x4096 11.7 / 14.9, 128x2048x4096 11.4 / 18.0, 64x64x8192
+//   12.2 / 16.4 (a tie where both run at HBM's rate: 32x8192x8192 29.4 / 29.1); two, while K is short: 64x8192x2048 14.1 / 17.3, x8192 50 / 33; four (16x32000x2048) 24.0 / 22.9.
+// - 16-bit, unaligned: 16x2001x2049 11.3 / 22.2, 64x2001x2001 10.3 / 20.7, 40x6001x1501 (two rounds)
+//   20.7 / 32.4; long K needs many columns: 16x4001x4097 19.8 / 41.6, 16x1001x4097 20.8 / 17.1,
+//   64x4097x4095 64 / 42.
+// - fp32 against the 128 x 128-tile kernel, whose one round takes six times as long: 256x4096x4096
+//   (four rounds) 133 / 298, 128x8192x512 24 / 41. Against the other fp32 forms up to 128 rows:
+//   128x1024x1024 6.8 / 10.9, 64x512x4096 16.4 / 34.1 (split K from 16 blocks on: its narrowest
+//   outputs keep the 32 x 32 blocks), but 256x1024x1024 13.4 / 11.5 and 2x65x8001 27.5 / 23.6.
+bool gemm_skinny_pays(long long M, long long N, long long K, bool f32, bool mfma, bool splitk) {
+  if (K < 64 || N < gemms::kCols) return false;  // nothing to gain: calls of a launch's length
+  const long long tiles = cdiv(N, gemms::kCols);
+  const long long rounds = cdiv(tiles * cdiv(M, gemm_skinny_rows(M, N)), kNumCUs);
+  if (f32 && mfma) return M <= 512 && rounds <= 4;
+  if (M > 128 || rounds > 2) return false;
+  if (f32) return splitk ? tiles * cdiv(M, 16) >= 16 : tiles >= 8 || K <= 4096;
+  if (mfma) return rounds == 1 || K <= 2048;
+  return K <= 2304 || (rounds == 1 && M <= 32 && tiles >= 60);
+}
+
 int matmul_impl(const KgArgSlot* args, unsigned long long n) {
   if (args == nullptr) return fail(kInvalid, "ordered_args is null");
   if (n != 4 && n != 7 && n != 8) return fail(kInvalid, "matmul expects 4, 7 or 8 slots, got %llu", n);
@@ -578,7 +603,10 @@ int matmul_impl(const KgArgSlot* args, unsigned long long n) {
   const bool simt = f32 ? !f32_mfma_ok && (!gemm_f32_splitk_ok(out, lhs, rhs, M, N, K) ||
                                            (bias.present && bias.stride[0] != 1))
                         : !mfma_ok;
-  const GemmPackedPlan packed = simt && !staged && gemm_packed_pays(M, N, K, f32) && lhs.stride[1] == 1 &&
+  const bool skinny = !staged && lhs.stride[1] == 1 && rhs.stride[1] == 1 &&
+                      out.stride[1] == 1 && lhs.stride[0] <= kMaxPipeLd && rhs.stride[0] <= kMaxPipeLd &&
+                      (!bias.present || bias.stride[0] == 1) && gemm_skinny_pays(M, N, K, f32, f32 ? f32_mfma_ok : mfma_ok, !simt);
+  const GemmPackedPlan packed = !skinny && simt && !staged && gemm_packed_pays(M, N, K, f32) && lhs.stride[1] == 1 &&
                                         rhs.stride[1] == 1 && out.stride[1] == 1 &&
                                         out.stride[0] <= 0x7fffffff && (!bias.present || bias.stride[0] == 1)
                                     ? gemm_packed_plan(M, N, K, f32, kSplitMaxWorkspace)
@@ -603,11 +631,28 @@ int matmul_impl(const KgArgSlot* args, unsigned long long n) {
         mfma = cdiv(M, gemmm::kT) * cdiv(N, gemmm::kT) * cdiv(K, gemmm::kBK) * 128;
       cyc = 16;
     }
+    if (skinny && M > 0) {  // per 16 rows x 32 columns and 32-deep step 2 (16x16x32), fp32 16 (16x16x4)
+      mfma = cdiv(M, gemm_skinny_rows(M, N)) * (gemm_skinny_rows(M, N) / 16) * cdiv(N, gemms::kCols) * cdiv(K, gemms::kStep) * (f32 ? 16 : 2);
+      cyc = f32 ? 32 : 16;
+    }
     const long long es = esize(out.dtype);
     return record_cost(M * N * K, mfma, cyc, (M * K + K * N) * es + (bias.present ? N * esize(bias.dtype) : 0),
                        M * N * es);
   }
   if (M == 0 || N == 0) return finish_launch("matmul(empty)");
+  if (skinny) {
+    const int bias_kind = !bias.present ? 0 : (bias.dtype == KG_DTYPE_F32 ? 1 : 2);
+    const void* bp = bias.present ? bias.data : nullptr;
+#define KG_GEMM_SKINNY(TAG)                                                                                         \
+  launch_gemm_skinny<TAG>(lhs.data, rhs.data, out.data, bp, bias_kind, m, nn, k, lhs.stride[0], rhs.stride[0], \
+                          out.stride[0], g_stream)
+    const hipError_t e = f32                          ? KG_GEMM_SKINNY(F32Tag)
+                         : out.dtype == KG_DTYPE_BF16 ? KG_GEMM_SKINNY(Bf16Tag)
+                                                      : KG_GEMM_SKINNY(F16Tag);
+#undef KG_GEMM_SKINNY
+    if (e != hipSuccess) return fail(kHipFailure, "matmul(skinny): %s", hipGetErrorString(e));
+    return finish_launch("matmul(skinny)");
+  }
   // (while a graph records, the workspace may not be used: it may be replaced later)
   if (packed_ok && !stream_capturing()) {
     SplitLease lease = split_workspace(packed.bytes(), g_stream);

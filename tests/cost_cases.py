@@ -11,7 +11,7 @@ dispatches are the HIP runtime's own copy kernels (named __amd_rocclr_*) that so
 host-to-device copies use, so leaving out those and the *_splitk_reduce_kernel, *_pack_kernel and *_combine_kernel dispatches,
 library dispatch i of the counter run is case i. Cases cover every kernel choice the model distinguishes: the
 pipelined MFMA GEMM with 256- and 128-row tiles and with ragged edges, the fp32 MFMA GEMM
-aligned and ragged, the fp32 split-K GEMM, the SIMT GEMM, the MFMA conv with four and with two live waves and a
+aligned and ragged, the fp32 split-K GEMM, the few-row GEMM, the SIMT GEMM, the MFMA conv with four and with two live waves and a
 ragged last row block, the implicit-GEMM conv (16-bit and fp32) and its row-piece form
 (16-bit 8- and 4-pixel pieces, 3x3 and 1x1, stride 1 and 2; fp32), and the 16-bit and fp32 MFMA attention kernels for D=128 and D=64,
 causal and not, with ragged query and key tails.
@@ -64,6 +64,8 @@ CASES = (
     ("fa_f32_causal_1x40x250x64", "flash_attention", "float32", ((1, 40, 250, 64),) * 4, (64, 64, 0.125, 1)),
     ("fa_bf16_2x3x100x80", "flash_attention", "bfloat16", ((2, 3, 100, 80),) * 4, (64, 64, 0.125, 1)),
     ("gemm_f16_packed_301x999x777", "matmul", "float16", ((301, 999), (301, 777), (777, 999)), ()),
+    ("gemm_bf16_skinny_16x4096x4096", "matmul", "bfloat16", ((16, 4096), (16, 4096), (4096, 4096)), ()),
+    ("gemm_f32_skinny_33x1001x777", "matmul", "float32", ((33, 777), (33, 1001), (1001, 777)), ()),
     ("fa_f32_2x1x130x64", "flash_attention", "float32", ((2, 1, 130, 64),) * 4, (64, 64, 0.125, 0)),
 )
 

@@ -597,3 +597,83 @@ def test_128_tiles_match_wide_tiles(device, shape, bias_kind, dtype_name):
         native.call_entry("kg_gfx950_matmul_entry", args)
         assert torch.equal(big[:m, :n], wide[:, :n]), f"stages={stages}"
         assert torch.isnan(big[m:]).all() and torch.isnan(big[:, n:]).all(), "store outside the output window"
+
+
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float16", "float32"])
+@pytest.mark.parametrize(
+    "shape,bias_kind,odd",
+    [
+        ((16, 4096, 4096), "f32", False),  # whole steps, 4 batches per wave
+        ((1, 64, 32), "none", False),  # one batch of one tile
+        ((3, 65, 33), "same", True),  # one k past a batch, one column past a tile
+        ((17, 1023, 95), "f32", True),  # one row past a block; the last step one short, odd N
+        ((33, 1089, 2049), "same", True),  # K one past 17 batches, the last pair shifted
+        ((64, 2112, 8200), "none", False),  # 32-row blocks, 257 tiles, one batch per wave and a second
+        ((128, 1120, 999), "same", True),  # 16-row blocks, K half a batch over
+        ((100, 160, 4100), "f32", True),  # 32-row blocks of a ragged M
+    ],
+)
+def test_few_rows(device, shape, bias_kind, odd, dtype_name):
+    """The few-row kernel against float64: an output is rounded once (bf16 2^-9, f16 2^-12 of it, fp32
+    covered by the sums) and its products are summed in fp32 in any order: at most k roundings of
+    2^-24 of sum |a b|. odd: operands and output are windows of wider buffers with odd row strides and bases;
+    nothing outside the output window is written. Rows of k past the end hold NaN."""
+
+    import torch
+
+    dt = getattr(torch, dtype_name)
+    m, k, n = shape
+    gen = torch.Generator(device=device).manual_seed(m + k + n)
+    pad = 1 if odd else 0
+    wide_a = torch.full((m + 1, k + 2 * pad), float("nan"), dtype=dt, device=device)
+    wide_b = torch.full((k + 1, n + 2 * pad), float("nan"), dtype=dt, device=device)
+    a, b = wide_a[:m, pad : pad + k], wide_b[:k, pad : pad + n]
+    a.copy_(torch.randn(m, k, generator=gen, device=device))
+    b.copy_(torch.randn(k, n, generator=gen, device=device))
+    bias = None if bias_kind == "none" else torch.randn(n, generator=gen, device=device)
+    if bias_kind == "same":
+        bias = bias.to(dt)
+    wide = torch.full((m + 1, n + 2 * pad), float("nan"), dtype=dt, device=device)
+    out = wide[:m, pad : pad + n]
+    print(f"[matmul] few rows {shape} {dtype_name}", flush=True)
+    native.matmul(out, a, b, bias)
+    ref, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    if bias is not None:
+        ref, size = ref + bias.double(), size + bias.double().abs()
+    half_ulp = {"bfloat16": 2.0**-9, "float16": 2.0**-12, "float32": 0.0}[dtype_name]
+    tol = (k + 2) * 2.0**-24 * size
+    tol = tol + half_ulp * 2 * (ref.abs() + tol)
+    assert ((out.double() - ref).abs() <= tol).all()
+    assert torch.isnan(wide[m:]).all()
+    if pad:
+        assert torch.isnan(wide[:, :pad]).all() and torch.isnan(wide[:, pad + n :]).all()
+
+
+@pytest.mark.parametrize("shape", [(5, 700, 333), (170, 1001, 99)], ids=["fewrows", "packed"])
+def test_matmul_under_capture(device, shape):
+    """A graph holds a few-row call (one launch, no workspace) and one whose packed form gives way to
+    the SIMT kernel; each replay reads its inputs anew."""
+
+    import torch
+
+    m, k, n = shape
+    a, b = torch.randn(m, k, device=device), torch.randn(k, n, device=device)
+    out, eager = torch.empty(m, n, device=device), torch.empty(m, n, device=device)
+    stream = torch.cuda.Stream(device=device)
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.graph(graph, stream=stream):
+            native.set_launch_mode(False, stream.cuda_stream)
+            native.matmul(out, a, b, None)
+    finally:
+        native.set_launch_mode(True, None)
+    for _ in range(3):
+        a.normal_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        tol = (k + 2) * 2.0**-24 * (a.double().abs() @ b.double().abs())
+        assert ((out.double() - a.double() @ b.double()).abs() <= tol).all()
+        native.matmul(eager, a, b, None)
+        assert ((eager.double() - out.double()).abs() <= 2 * tol).all()
