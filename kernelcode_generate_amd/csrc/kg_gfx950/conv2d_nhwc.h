@@ -114,7 +114,7 @@ __global__ __launch_bounds__(convn::kThreads) void conv_pack_kernel(
     const uint32_t n = fdiv(row, s.div_hp);
     if ((int)n >= s.n) return;
     const int hi = (int)(row - n * s.hp) * s.row_step - s.pt;
-    const int hw = s.h * s.w;
+    const long long hw = (long long)s.h * s.w;  // (a plane may have 2^31 elements: only the copy is bounded)
     const int c0 = (int)cb * V;
     u32x4 in[V], out[V];
 #pragma unroll
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(convn::kThreads) void conv_pack_kernel(
       const long long last = (long long)s.n * s.c * hw - V;
 #pragma unroll
       for (int e = 0; e < V; ++e) {
-        const long long at = first + (long long)e * hw;
+        const long long at = first + e * hw;
         if (c0 + e < s.c) {
           if (at >= 0 && at <= last) {
             in[e] = ld16_any(x + at);

@@ -378,3 +378,30 @@ def test_channel_last_matches_gather(device, dtype_name, xs, ws, stride, dil, pa
     flat[torch.randint(0, flat.numel(), (7,), generator=gen, device=device)] = float("inf")
     got, ref = conv(x, w, b, None), conv(x, w, b, 2)
     assert torch.equal(torch.isfinite(got), torch.isfinite(ref)) and not torch.isfinite(ref).all()
+
+
+def test_channel_last_planes_beyond_int32(device):
+    """An image plane of more than 2^31 elements of which the windows touch one row: the copy is
+    small, but a channel's plane starts beyond a 32-bit offset. Reference and bar as
+    test_channel_last_matches_gather's, in float64 over the touched row."""
+
+    import torch
+
+    h, w, f, kw = 2050, 1048000, 8, 49
+    wo, k = w - kw + 1, 2 * kw
+    assert h * w > 2**31
+    specs = [native.TensorSpec(s, "bfloat16") for s in ((1, f, 1, wo), (1, 2, h, w), (f, 2, 1, kw))]
+    model = native.cost("conv2d", [*specs, None, h, 1, 1, 1, 0, 0, 0, 0])
+    assert model["MFMA"] > 0 and model["MFMA_CYCLES"] == model["MFMA"] * 16  # the route under test
+    gen = torch.Generator(device=device).manual_seed(5)
+    x = torch.zeros(1, 2, h, w, dtype=torch.bfloat16, device=device)
+    x[:, :, 0] = torch.randn(1, 2, w, generator=gen, device=device)
+    wt = torch.randn(f, 2, 1, kw, generator=gen, device=device).bfloat16()
+    out = torch.full((1, f, 1, wo), float("nan"), dtype=torch.bfloat16, device=device)
+    print("[conv2d] a plane of 2050 x 1048000", flush=True)
+    native.conv2d(out, x, wt, None, (h, 1), (1, 1), (0, 0, 0, 0))
+    cols = x[0, :, 0].double().unfold(1, kw, 1).permute(0, 2, 1).reshape(k, wo)
+    weights = wt.double().reshape(f, k)
+    ref, terms = weights @ cols, weights.abs() @ cols.abs()
+    tol = 2.0**-8 * ref.abs() + 2.0**-24 + 8 * k**0.5 * 2.0**-24 * terms
+    assert ((out[0, :, 0].double() - ref).abs() <= tol).all()
