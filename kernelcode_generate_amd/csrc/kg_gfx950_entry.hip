@@ -293,8 +293,11 @@ int pipe_splits(long long M, long long N, long long K, long long* chunk) {
 // call is between its two launches) and releases its buffer with hipFree, which waits for
 // the device's pending work (the stream the buffer was used on may no longer exist). Lock
 // order: the table's mutex, then a slot's. An allocation per call (hipMallocAsync /
-// hipFreeAsync) cost about 60 us of host time per matmul. Calls that split allocate on the
-// first use per stream (or a larger shape): they are not capturable in a HIP graph then.
+// hipFreeAsync) cost about 60 us of host time per matmul.
+// While the stream records a graph there is no workspace: the graph would keep the buffer's
+// address beyond its replacement by any later call on that stream, and allocating invalidates
+// the recording. Every caller then takes its form without one: K or the keys not split, the
+// gathering conv, the SIMT matmul.
 constexpr int kSplitCachedStreams = 8;
 struct SplitWorkspace {
   int device;
@@ -312,11 +315,10 @@ std::mutex g_split_ws_mutex;
 std::vector<SplitWorkspace> g_split_ws;
 unsigned long long g_split_ws_clock = 0;
 
-// True while the calling thread's stream records a graph (or cannot be asked because another
-// stream does).
-bool stream_capturing() {
+// True while `stream` records a graph (or cannot be asked because another stream does).
+bool stream_capturing(hipStream_t stream) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(g_stream, &status) != hipSuccess) {
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
     (void)hipGetLastError();
     return true;
   }
@@ -325,6 +327,7 @@ bool stream_capturing() {
 
 SplitLease split_workspace(size_t bytes, hipStream_t stream) {
   SplitLease lease;
+  if (stream_capturing(stream)) return lease;
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) return lease;
   std::lock_guard<std::mutex> lock(g_split_ws_mutex);
@@ -653,8 +656,7 @@ int matmul_impl(const KgArgSlot* args, unsigned long long n) {
     if (e != hipSuccess) return fail(kHipFailure, "matmul(skinny): %s", hipGetErrorString(e));
     return finish_launch("matmul(skinny)");
   }
-  // (while a graph records, the workspace may not be used: it may be replaced later)
-  if (packed_ok && !stream_capturing()) {
+  if (packed_ok) {
     SplitLease lease = split_workspace(packed.bytes(), g_stream);
     if (char* ws = static_cast<char*>(lease.ptr)) {
       const int bias_kind = !bias.present ? 0 : (bias.dtype == KG_DTYPE_F32 ? 1 : 2);
@@ -855,10 +857,10 @@ int conv2d_impl(const KgArgSlot* args, unsigned long long n) {
     return finish_launch("conv2d(rowvec)");
   }
   // Everything else: the channel-last copy and its GEMM, or, for tiny calls, a set stage count
-  // (that kernel's ring is its own), while a graph records (its workspace may be replaced
-  // later) and where the copy does not fit the workspace, the gathering implicit GEMM.
+  // (that kernel's ring is its own), without a workspace (while a graph records) and where the
+  // copy does not fit it, the gathering implicit GEMM.
   if (const ConvNhwcPlan plan = conv_nhwc_plan(s, out.dtype == KG_DTYPE_F32, kSplitMaxWorkspace);
-      plan.ok && !staged && aligned16(out.data) && !stream_capturing()) {
+      plan.ok && !staged && aligned16(out.data)) {
     lease = split_workspace(plan.bytes(), g_stream);
     if (char* ws = static_cast<char*>(lease.ptr)) {
       const int bias_kind = !bias.present ? 0 : (bias.dtype == KG_DTYPE_F32 ? 1 : 2);
@@ -1031,12 +1033,11 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
   }
 
   if (decode) {
-    // one range per (b,h) where there is no workspace, or while a graph records (it may be
-    // replaced later)
+    // one range per (b,h) where there is no workspace (while a graph records)
     FaDecodePlan plan = fa_decode_plan(s, f32, true);
     SplitLease lease;
     if (plan.splits > 1) {
-      if (!stream_capturing()) lease = split_workspace(plan.bytes, g_stream);
+      lease = split_workspace(plan.bytes, g_stream);
       if (lease.ptr == nullptr) plan = fa_decode_plan(s, f32, false);
     }
     float* partial = static_cast<float*>(lease.ptr);

@@ -1,0 +1,246 @@
+"""The per-stream workspace of the calls that take one (kg_gfx950_entry.hip, split_workspace): the
+fp32 partial sums of a K split over workgroups, packed operands, a conv's channel-last copy, the
+partial outputs of split keys. One call of each kind, its route checked by its cost record, is run
+from two threads on one stream, on more streams than buffers are kept for, with buffers that are
+replaced by larger ones meanwhile, and under graph capture.
+A call's sums are in a fixed order, so its bits are compared with those of a call by itself."""
+
+from __future__ import annotations
+
+import threading
+
+import pytest
+
+from kernelcode_generate_amd import native
+from tests.gpu_util import assert_f32_close, assert_h16_close, to_numpy
+
+pytestmark = pytest.mark.gpu
+
+# name: (operation, dtype, sizes, MFMA instructions of the route meant)
+CALLS = {
+    # matmul (M, K, N): 3 tiles of 128 x 256 and 46 slices of 32, in 5 K chunks
+    "matmul_split": ("matmul", "bfloat16", (371, 1472, 256), 3 * 46 * 128),
+    # 12 tiles of 128 x 256 and 80 slices, in 10 chunks (15.7 MB of partials)
+    "matmul_split_large": ("matmul", "bfloat16", (384, 2560, 1024), 12 * 80 * 128),
+    # odd rows: 6 tiles of 64 x 64 and 63 slices of 64, in 7 chunks
+    "matmul_packed": ("matmul", "float16", (170, 4001, 99), 6 * 63 * 32),
+    "matmul_packed_f32": ("matmul", "float32", (170, 4001, 99), 6 * 126 * 128),
+    # conv (images, filters, stride, pad, memory_stage): the row-piece kernel, 14 tiles of 64 x 128, split
+    "conv_rowvec": ("conv2d", "float16", ((1, 128, 28, 28), (128, 128, 3, 3), 1, 1, None), 7 * 24 * 16 * 3),
+    # the gathering kernel (a set stage count), 4 tiles and 144 slices, in 36 chunks
+    "conv_gather": ("conv2d", "bfloat16", ((2, 512, 7, 7), (512, 512, 3, 3), 1, 1, 2), 4 * 144 * 4 * 2 * 2 * 2),
+    # the channel-last copy, 8 tiles of 64 x 64 and 45 slices, split; 1568 of 128 x 64 and 4 slices (13.5 MB)
+    "conv_copy": ("conv2d", "bfloat16", ((2, 300, 15, 15), (64, 300, 3, 3), 1, 1, None), 8 * 45 * 32),
+    "conv_copy_large": ("conv2d", "float16", ((16, 3, 224, 224), (64, 3, 7, 7), 2, 3, None), 1568 * 4 * 64),
+    # attention (B, H, S_q, S_kv, D): 8 heads of one query and 128 steps of 32 keys, 16 ranges of keys
+    "attention_bf16": ("attention", "bfloat16", (1, 8, 1, 4096, 128), 8 * 128 * 17),
+    "attention_f32": ("attention", "float32", (1, 2, 16, 2000, 64), 2 * 125 * 32),
+}
+NAMES = [n for n in CALLS if not n.endswith("_large")]
+
+
+def make(name, device, seed=0):
+    """(call, output shape, dtype) of CALLS[name]: call(out) runs it on fixed inputs."""
+
+    import torch
+
+    op, dtype_name, size, mfma = CALLS[name]
+    dt = getattr(torch, dtype_name)
+    gen = torch.Generator(device=device).manual_seed(seed + len(name))
+
+    def draw(*shape, scale=1.0):
+        return (torch.randn(shape, generator=gen, device=device) * scale).to(dt)
+
+    if op == "matmul":
+        m, k, n = size
+        args = (draw(m, k), draw(k, n, scale=k**-0.5), draw(n))
+        shape, scalars = (m, n), ()
+        entry = "kg_gfx950_matmul_entry"
+    elif op == "conv2d":
+        xs, ws, stride, pad, stage = size
+        args = (draw(*xs), draw(*ws, scale=(ws[1] * ws[2] * ws[3]) ** -0.5), draw(ws[0]))
+        side = [(xs[i] + 2 * pad - ws[i]) // stride + 1 for i in (2, 3)]
+        shape = (xs[0], ws[0], *side)
+        scalars = (stride, stride, 1, 1, pad, pad, pad, pad) + (() if stage is None else (1, 1, 1, 1, 1, stage))
+        entry = "kg_gfx950_conv2d_entry"
+    else:
+        b, h, s_q, s_kv, d = size
+        args = (draw(b, h, s_q, d), draw(b, h, s_kv, d), draw(b, h, s_kv, d))
+        shape, scalars = (b, h, s_q, d), (64, 64, d**-0.5, 0)
+        entry = "kg_gfx950_flash_attention_entry"
+    family = {"attention": "flash_attention"}.get(op, op)
+    specs = [native.TensorSpec(shape, dtype_name), *(native.TensorSpec.of(a) for a in args)]
+    model = native.cost(family, [*specs, *scalars])
+    assert model["MFMA"] == mfma, f"{name} takes another route: {model['MFMA']} MFMAs"
+    torch.cuda.synchronize()
+
+    def call(out):
+        native.call_entry(entry, (out, *args, *scalars))
+
+    return call, shape, dt
+
+
+def alone(name, device, seed=0):
+    """(call, a function that makes an output, the call's result by itself)."""
+
+    import torch
+
+    call, shape, dt = make(name, device, seed)
+
+    def output():
+        return torch.full(shape, float("nan"), dtype=dt, device=device)
+
+    expected = output()
+    torch.cuda.synchronize()
+    native.set_launch_mode(True, None)
+    call(expected)
+    assert torch.isfinite(expected).all()
+    return call, output, expected
+
+
+def run_threads(workers):
+    errors: list[BaseException] = []
+    start = threading.Barrier(len(workers))
+
+    def guarded(worker):
+        try:
+            start.wait()
+            worker()
+        except BaseException as exc:  # noqa: BLE001 - reported by the main thread
+            errors.append(exc)
+
+    threads = [threading.Thread(target=guarded, args=(w,)) for w in workers]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=100)
+    assert not any(t.is_alive() for t in threads), "a worker did not finish"
+    assert not errors, errors
+
+
+@pytest.mark.parametrize(
+    "first,second",
+    [("matmul_split", "conv_copy"), ("matmul_packed", "attention_bf16"), ("conv_rowvec", "matmul_packed_f32"),
+     ("conv_gather", "attention_f32"), ("conv_copy", "conv_rowvec")],
+)
+def test_two_threads_on_one_stream(device, first, second):
+    """Two synchronous threads on the default stream: a call's launches are not parted by another
+    call that writes the same workspace."""
+
+    import torch
+
+    made = [alone(n, device) for n in (first, second)]
+    wrong: list[tuple[str, int]] = []
+
+    def worker(name, call, output, expected):
+        native.set_launch_mode(True, None)
+        for r in range(30):
+            out = output()
+            call(out)
+            if not torch.equal(out, expected):
+                wrong.append((name, r))
+
+    print(f"[workspace] two threads: {first}, {second}", flush=True)
+    run_threads([lambda n=n, m=m: worker(n, *m) for n, m in zip((first, second), made)])
+    assert not wrong, wrong
+
+
+def test_larger_requests_from_another_thread(device):
+    """On each of ten streams one thread enqueues small calls while another's calls ask for ever
+    larger workspaces, so a buffer with work still enqueued on it is replaced."""
+
+    import torch
+
+    small = alone("matmul_split", device)
+    growing = [alone(n, device) for n in ("attention_bf16", "conv_copy", "conv_copy_large", "matmul_split_large")]
+    for trial in range(10):
+        stream = torch.cuda.Stream(device=device)
+        small_out = [small[1]() for _ in range(12)]
+        growing_out = [m[1]() for m in growing]
+        torch.cuda.synchronize()
+        print(f"[workspace] growing requests, stream {trial}", flush=True)
+
+        def enqueue(calls):
+            native.set_launch_mode(False, stream.cuda_stream)
+            for call, out in calls:
+                call(out)
+
+        run_threads([lambda: enqueue([(small[0], o) for o in small_out]),
+                     lambda: enqueue([(m[0], o) for m, o in zip(growing, growing_out)])])
+        torch.cuda.synchronize()
+        for out in small_out:
+            assert torch.equal(out, small[2]), f"trial {trial}"
+        for m, out in zip(growing, growing_out):
+            assert torch.equal(out, m[2]), f"trial {trial}"
+
+
+def test_more_streams_than_buffers(device):
+    """Two rounds over 11 streams, every kind of call on each: the ninth and later streams take
+    over the least recently used buffer (8 are kept per device)."""
+
+    import torch
+
+    streams = [torch.cuda.Stream(device=device) for _ in range(11)]
+    made = {n: alone(n, device) for n in NAMES}
+    results = []
+    outputs = {(r, i, n): made[n][1]() for r in range(2) for i in range(len(streams)) for n in NAMES}
+    torch.cuda.synchronize()
+    try:
+        for rnd in range(2):
+            for i, stream in enumerate(streams):
+                print(f"[workspace] round {rnd} stream {i}", flush=True)
+                native.set_launch_mode(False, stream.cuda_stream)
+                for n in NAMES:
+                    out = outputs[rnd, i, n]
+                    made[n][0](out)
+                    results.append((rnd, i, n, out))
+    finally:
+        native.set_launch_mode(True, None)
+    torch.cuda.synchronize()
+    for rnd, i, n, out in results:
+        assert torch.equal(out, made[n][2]), f"{n}, round {rnd} stream {i}"
+
+
+@pytest.mark.parametrize("warm", [True, False], ids=["warm", "cold"])
+@pytest.mark.parametrize("name", NAMES)
+def test_captured_calls_keep_no_workspace(device, name, warm):
+    """A graph recorded on a stream, one that has a workspace (warm) or one that has not (where
+    allocating would invalidate the recording), holds none of it: after a larger call on that
+    stream has replaced the buffer, and others have written to the new one, every replay gives the
+    call's result (in another order of sums: the call's K or keys are not split)."""
+
+    import torch
+
+    call, output, expected = alone(name, device)
+    larger, larger_output, larger_expected = alone("conv_copy_large", device)
+    stream = torch.cuda.Stream(device=device)
+    eager, out, big = output(), output(), larger_output()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    try:
+        native.set_launch_mode(False, stream.cuda_stream)
+        if warm:
+            call(eager)
+            stream.synchronize()
+        print(f"[workspace] capture {name} warm={warm}", flush=True)
+        with torch.cuda.graph(graph, stream=stream):
+            native.set_launch_mode(False, stream.cuda_stream)
+            call(out)
+        native.set_launch_mode(False, stream.cuda_stream)
+        larger(big)
+        stream.synchronize()
+        assert torch.equal(big, larger_expected) and (not warm or torch.equal(eager, expected))
+        close = assert_f32_close if out.dtype == torch.float32 else assert_h16_close
+        first = None
+        for _ in range(3):
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            larger(big)
+            call(eager)
+            torch.cuda.synchronize()
+            close(to_numpy(out), to_numpy(expected), what=f"replay of {name}")
+            first = out.clone() if first is None else first
+            assert torch.equal(out, first) and torch.equal(eager, expected) and torch.equal(big, larger_expected)
+    finally:
+        native.set_launch_mode(True, None)
