@@ -325,6 +325,23 @@ bool stream_capturing(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
+// Allocating is refused, and invalidates the recording, while any other thread records a graph
+// in the global mode, unless the allocating thread is in the relaxed one: its buffers are not
+// part of that graph.
+class RelaxedCaptureMode {
+ public:
+  RelaxedCaptureMode() { swap(); }
+  ~RelaxedCaptureMode() { swap(); }
+  RelaxedCaptureMode(const RelaxedCaptureMode&) = delete;
+  RelaxedCaptureMode& operator=(const RelaxedCaptureMode&) = delete;
+
+ private:
+  void swap() {
+    if (hipThreadExchangeStreamCaptureMode(&mode_) != hipSuccess) (void)hipGetLastError();
+  }
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 SplitLease split_workspace(size_t bytes, hipStream_t stream) {
   SplitLease lease;
   if (stream_capturing(stream)) return lease;
@@ -347,6 +364,7 @@ SplitLease split_workspace(size_t bytes, hipStream_t stream) {
       return lease;
     }
   }
+  const RelaxedCaptureMode relaxed;
   void* ptr = nullptr;
   const size_t want = std::max(bytes, (size_t)(4u << 20));
   if (hipMalloc(&ptr, want) != hipSuccess) {

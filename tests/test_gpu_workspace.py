@@ -2,7 +2,7 @@
 fp32 partial sums of a K split over workgroups, packed operands, a conv's channel-last copy, the
 partial outputs of split keys. One call of each kind, its route checked by its cost record, is run
 from two threads on one stream, on more streams than buffers are kept for, with buffers that are
-replaced by larger ones meanwhile, and under graph capture.
+replaced by larger ones meanwhile, under graph capture, and while another thread records a graph.
 A call's sums are in a fixed order, so its bits are compared with those of a call by itself."""
 
 from __future__ import annotations
@@ -244,3 +244,45 @@ def test_captured_calls_keep_no_workspace(device, name, warm):
             assert torch.equal(out, first) and torch.equal(eager, expected) and torch.equal(big, larger_expected)
     finally:
         native.set_launch_mode(True, None)
+
+
+def test_first_call_while_another_thread_records(device):
+    """A stream's first call that takes a workspace, made while another thread records a graph (in
+    the mode that refuses other threads' allocations): the call's bits are those it has otherwise,
+    and the recording is not disturbed."""
+
+    import torch
+
+    streams = [torch.cuda.Stream(device=device) for _ in range(11)]
+    call, output, expected = alone("matmul_packed_f32", device)
+    recorded, recorded_output, recorded_expected = alone("matmul_split", device)
+    fresh, recording = streams[0], streams[10]
+    for s in streams[1:10]:  # nine other streams: whatever buffer `fresh` had has gone to one of them
+        out = output()
+        torch.cuda.synchronize()
+        native.set_launch_mode(False, s.cuda_stream)
+        call(out)
+        s.synchronize()
+    out, graph_out = output(), recorded_output()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    print("[workspace] a first call while another thread records", flush=True)
+    try:
+        with torch.cuda.graph(graph, stream=recording):
+            native.set_launch_mode(False, recording.cuda_stream)
+            recorded(graph_out)
+
+            def worker():
+                native.set_launch_mode(False, fresh.cuda_stream)
+                call(out)
+
+            run_threads([worker])
+    finally:
+        native.set_launch_mode(True, None)
+    torch.cuda.synchronize()
+    assert torch.equal(out, expected)
+    for _ in range(3):
+        graph_out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_h16_close(to_numpy(graph_out), to_numpy(recorded_expected), what="replay")
