@@ -361,16 +361,18 @@ __global__ __launch_bounds__(convn::kThreads, 2) void conv2d_nhwc_kernel(
     static_for<kSteps>([&](auto idx_tag) __attribute__((always_inline)) {
       constexpr int idx = decltype(idx_tag)::value;
       constexpr int ks = idx / (MA * NB), i = idx % (MA * NB) / NB, j = idx % NB;
-      if constexpr (kHalves && idx % (MA * NB) == 0) {
+      if constexpr (V == 8 && idx % (MA * NB) == 0) {
         // paired pixels: an odd kernel row ends in the middle of a chunk, and the pixel after it
         // (any value, infinities included) must not meet the weights' zeros
-        const uint32_t h = 2 * (kt0 + it) + ks;
-        const int in_run = (int)(h - fdiv31(h, s.div_hpr) * s.hpr);
-        const uint32_t keep = s.paired && (s.kw & 1) && 4 * in_run + lg == s.cpr - 1 ? 0u : ~0u;
+        if (s.paired && (s.kw & 1)) {
+          const uint32_t u = kHalves ? 2 * (kt0 + it) + ks : kt0 + it;  // this step's half, this slice
+          const int in_run = (int)(u - fdiv31(u, kHalves ? s.div_hpr : s.div_spr) * units);
+          const uint32_t keep = (kHalves ? 4 * in_run : 8 * in_run + 4 * ks) + lg == s.cpr - 1 ? 0u : ~0u;
 #pragma unroll
-        for (int b = 0; b < MA; ++b) {
-          af[ks][b][2] &= keep;
-          af[ks][b][3] &= keep;
+          for (int b = 0; b < MA; ++b) {
+            af[ks][b][2] &= keep;
+            af[ks][b][3] &= keep;
+          }
         }
       }
       if constexpr (V == 8) {

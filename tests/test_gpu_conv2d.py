@@ -326,6 +326,9 @@ def test_rejects_bad_params(device):
         ((8, 3, 121, 115), (53, 3, 7, 7), (2, 2), (1, 1), (3, 3, 3, 3), "same"),  # paired pixels, rows end mid-chunk
         ((9, 4, 80, 90), (70, 4, 7, 4), (2, 2), (1, 1), (3, 3, 2, 1), None),  # paired pixels, even KW
         ((4, 3, 101, 95), (53, 3, 7, 7), (1, 1), (1, 1), (3, 3, 3, 3), "f32"),  # 3 channels, stride 1
+        ((8, 3, 121, 115), (53, 3, 9, 9), (2, 2), (1, 1), (4, 4, 4, 4), "f32"),  # paired pixels in runs of 5 chunks
+        ((8, 3, 151, 147), (64, 3, 11, 11), (4, 4), (1, 1), (2, 2, 2, 2), "same"),  # and of 6
+        ((3, 4, 151, 99), (64, 4, 19, 21), (2, 2), (1, 1), (9, 9, 10, 10), None),  # and of 11: two slices a run
         ((8, 17, 30, 33), (65, 17, 3, 3), (1, 1), (2, 2), (2, 2, 2, 2), "same"),  # dilated: runs are taps
         ((2, 130, 29, 29), (129, 130, 3, 3), (2, 1), (1, 2), (1, 0, 2, 1), "f32"),  # dilated columns, ragged everywhere
         ((9, 390, 21, 23), (72, 390, 1, 1), (1, 1), (1, 1), (0, 0, 0, 0), None),  # one tap
@@ -335,7 +338,7 @@ def test_rejects_bad_params(device):
         ((8, 3, 112, 111), (192, 3, 7, 7), (2, 2), (1, 1), (3, 3, 3, 3), "f32"),  # 128-pixel tiles, short K
         ((6, 64, 301, 301), (8, 64, 3, 3), (1, 1), (1, 1), (1, 1, 1, 1), "same"),  # several passes over the batch
     ],
-    ids=["c20", "paired7", "paired4", "c3s1", "dil2", "dilw2", "tap1", "halves5", "split", "bm128", "bm128_shortk", "passes"],
+    ids=["c20", "paired7", "paired4", "c3s1", "paired9", "paired11", "paired21", "dil2", "dilw2", "tap1", "halves5", "split", "bm128", "bm128_shortk", "passes"],
 )
 def test_channel_last_matches_gather(device, dtype_name, xs, ws, stride, dil, pad, bias):
     """The channel-last form against the gathering implicit GEMM (which a call that sets its
