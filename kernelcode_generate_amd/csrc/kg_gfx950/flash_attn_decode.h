@@ -1,5 +1,7 @@
-// Attention of few queries against many keys (a decoding step): 16-bit Q/K/V/O [B,H,S,D],
-// queries in blocks of 16, D in {64, 128}, fp32 online softmax, no mask.
+// Attention with the keys of a (b,h) split over workgroups, queries in blocks of 16, fp32 online
+// softmax, Q/K/V/O [B,H,S,D]: 16-bit calls of few queries with D = 64 or 128 (a decoding step; no
+// mask), 16-bit calls of other head dims (multiples of 8, causal or not), and fp32 calls
+// (fa_split_f32_kernel below).
 //
 // Such a call reads K and V once and does little else, so what bounds it is how much of the
 // chip keeps loads in flight. fa_fwd_mfma_kernel gives a (b,h) one workgroup (B H = 128: half
@@ -37,7 +39,10 @@ constexpr float kMinMax = -3.0e38f;
 
 // splits == 1: O is written; else partial[(bh splits + split) s_q + q][D + 2] takes O (not
 // normalised), m (log2 units) and l.
-// kAny: head dims d < D (multiples of 8, rows padded with zeros in registers) and causal calls.
+// kAny: head dims d < D (multiples of 8, rows padded with zeros in registers), causal or not. No tiled
+// kernel has these dims, and the SIMT kernel keeps its probabilities in fp32: so does this form,
+// whose P V and row sums are fp32 products (v_mfma_f32_16x16x4_f32). They take sixteen times the
+// MFMA time of the 16-bit ones and bound it.
 template <typename Tag, int D, bool kAny>
 __global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint16_t* __restrict__ Q,
                                                                      const uint16_t* __restrict__ K,
@@ -137,28 +142,45 @@ __global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint1
 #pragma unroll
       for (int c = 0; c < NE; ++c) o[c] *= alpha;
     }
+    if constexpr (kAny) {
+      // P stays fp32 and V's elements are widened: MFMA (kb, i) contracts keys 16kb + 4(l/16) + i
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      u32x4 pp;  // keys 32c + 4 lr + 0..3, then + 16
+      for (int kb = 0; kb < 2 * NC; ++kb)
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+        for (int i = 0; i < 4; ++i) {
+          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf((float)sc[kb][i], scale_log2, -m_run));
+          l_run[0] += p;
+          const VRow row = b.v[kb >> 1][4 * (kb & 1) + i];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[2 * c + h][2 * q], scale_log2, -m_run));
-          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[2 * c + h][2 * q + 1], scale_log2, -m_run));
-          pp[2 * h + q] = H::pack2(p0, p1);
+          for (int e = 0; e < NE; ++e) {
+            const uint32_t pair = row[e >> 1];
+            o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(H::to_float((e & 1) ? pair >> 16 : pair & 0xffffu), p, o[e], 0, 0, 0);
+          }
         }
+    } else {
 #pragma unroll
-      for (int e = 0; e < NE; ++e) {  // column e of each lane's 8 rows
-        u32x4 vt;
+      for (int c = 0; c < NC; ++c) {
+        u32x4 pp;  // keys 32c + 4 lr + 0..3, then + 16
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t x = b.v[c][2 * q][e >> 1], y = b.v[c][2 * q + 1][e >> 1];
-          vt[q] = (e & 1) ? hi_halves(x, y) : lo_halves(x, y);
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[2 * c + h][2 * q], scale_log2, -m_run));
+            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[2 * c + h][2 * q + 1], scale_log2, -m_run));
+            pp[2 * h + q] = H::pack2(p0, p1);
+          }
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {  // column e of each lane's 8 rows
+          u32x4 vt;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t x = b.v[c][2 * q][e >> 1], y = b.v[c][2 * q + 1][e >> 1];
+            vt[q] = (e & 1) ? hi_halves(x, y) : lo_halves(x, y);
+          }
+          o[e] = H::mfma16(vt, pp, o[e]);
         }
-        o[e] = H::mfma16(vt, pp, o[e]);
+        l_run = H::mfma16(ones, pp, l_run);
       }
-      l_run = H::mfma16(ones, pp, l_run);
     }
   };
 
@@ -188,7 +210,12 @@ __global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint1
     compute(b0, key, false);
   }
 
-  // ---- combine the waves ----
+  // ---- combine the waves (kAny: first the four lane rows' keys of the row sum) ----
+  if constexpr (kAny) {
+    float l0 = l_run[0], l1 = l0;
+    fa::rows4_combine<false>(l0, l1);
+    l_run[0] = l0;
+  }
   if (l16 < nq) {
 #pragma unroll
     for (int e = 0; e < NE; ++e)
@@ -436,8 +463,8 @@ inline bool fa_decode_supported(const FaShape& s) {
 }
 // Head dims the tiled kernels do not have, which otherwise run one workgroup per query (16-bit:
 // multiples of 8 from 24, fp32: of 4; causal or not), any call (us, this kernel /
-// fa_fwd_simt_kernel: 16x389x389x80 fp32 26 / 139, bf16 9.5 / 104; 128x512x512x96 causal bf16 48 /
-// 775). Below 24 the padding to 64 is most of the work. And fp32 with D = 64 or 128, causal or not, of up
+// fa_fwd_simt_kernel: 16x389x389x80 fp32 24 / 131, bf16 16.9 / 102; 128x512x512x96 causal bf16 81 /
+// 779; 32x1x2048x96 bf16 11.2 / 103). Below 24 the padding to 64 is most of the work. And fp32 with D = 64 or 128, causal or not, of up
 // to 16 queries or 512 blocks of them, where fa_fwd_f32_mfma_kernel's blocks of 128 queries leave
 // CUs idle (8x1x8192x128 23 / 1179; 16x512x512x64 22 / 47; 24x64x64x64 10.5 / 9.5, x128 10.7 / 13.5;
 // 256x64x64x64, 1024 blocks, 11.9 / 9.4; 32x1024x1024x64, 2048 blocks, 151 / 95).
@@ -466,10 +493,16 @@ inline FaDecodePlan fa_decode_plan(const FaShape& s, bool f32, bool may_split) {
   return FaDecodePlan{(int)splits, (int)(per * step * fad::kWaves),
                       splits > 1 ? (size_t)s.bh * splits * s.s_q * (cols + 2) * sizeof(float) : 0};
 }
+// 16-bit calls of the kAny form (D = 64 and 128 come here without a mask only).
+inline bool fa_decode_any(const FaShape& s) { return s.causal || (s.d != 64 && s.d != 128); }
+
 // MFMA instructions: per step and block of queries 2 S^T blocks x D/32 and D/16 + 1 for O^T and the
-// row sums per 32 keys; fp32 4 for S^T and 4 for O^T per 16 d and 16 keys. Causal blocks stop at
-// their last query's step.
-inline long long fa_decode_mfma(const FaShape& s, bool f32, const FaDecodePlan& plan) {
+// row sums per 32 keys (other head dims: 8 fp32 ones x D/16 for O^T, counted apart); fp32 4 for S^T
+// and 4 for O^T per 16 d and 16 keys. Causal blocks stop at their last query's step.
+struct FaDecodeMfma {
+  long long h16, f32;  // v_mfma_f32_16x16x32 (16 cycles), v_mfma_f32_16x16x4_f32 (32 cycles)
+};
+inline FaDecodeMfma fa_decode_mfma(const FaShape& s, bool f32, const FaDecodePlan& plan) {
   const int step = f32 ? 16 : s.d > 64 ? fad::step_keys<128>() : fad::step_keys<64>();
   const int D = s.d > 64 ? 128 : 64, NE = s.d <= 64 ? 4 : s.d <= 96 ? 6 : 8;
   long long steps = 0;
@@ -478,7 +511,10 @@ inline long long fa_decode_mfma(const FaShape& s, bool f32, const FaDecodePlan& 
     for (long long lo = 0; lo < end; lo += plan.split_keys)
       steps += (std::min<long long>(plan.split_keys, end - lo) + step - 1) / step;
   }
-  return s.bh * steps * (f32 ? 8 * NE : (step / 32) * (D / 16 + D / 16 + 1));
+  const long long chunks = s.bh * steps * (step / 32);
+  if (f32) return FaDecodeMfma{0, s.bh * steps * 8 * NE};
+  if (fa_decode_any(s)) return FaDecodeMfma{chunks * (D / 16), chunks * 8 * (D / 16)};
+  return FaDecodeMfma{chunks * (D / 16 + D / 16 + 1), 0};
 }
 
 template <typename Tag, int D, bool kAny>
@@ -496,7 +532,7 @@ hipError_t launch_fa_decode_d(const uint16_t* q, const uint16_t* k, const uint16
 template <typename Tag>
 hipError_t launch_fa_decode(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* o, const FaShape& s,
                             const FaDecodePlan& plan, float* partial, hipStream_t stream) {
-  if (s.causal || (s.d != 64 && s.d != 128)) {
+  if (fa_decode_any(s)) {
     if (s.d > 64) return launch_fa_decode_d<Tag, 128, true>(q, k, v, o, s, plan, partial, stream);
     return launch_fa_decode_d<Tag, 64, true>(q, k, v, o, s, plan, partial, stream);
   }

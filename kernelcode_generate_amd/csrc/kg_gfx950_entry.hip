@@ -1013,8 +1013,9 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
     // products Q.K^T and P.V that the mask keeps: causal row i sees keys 0..i
     const long long pairs = s.causal ? (long long)s.s_q * (s.s_q + 1) / 2 : (long long)s.s_q * s.s_kv;
     long long mfma = 0;
+    FaDecodeMfma split = {0, 0};
     if (decode) {
-      mfma = fa_decode_mfma(s, f32, fa_decode_plan(s, f32, true));
+      split = fa_decode_mfma(s, f32, fa_decode_plan(s, f32, true));
     } else if ((out.dtype == KG_DTYPE_BF16 || out.dtype == KG_DTYPE_F16) && fa_mfma_supported(s) && out.numel() > 0) {
       // per workgroup: waves x key tiles x (D/4 16x16x32 MFMAs for S^T + D/4 for PV + 4 row sums)
       const int waves = fa_mfma_waves(s);
@@ -1046,8 +1047,10 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
       mfma = B_H * waves_tiles * s.d;
     }
     const long long es = esize(out.dtype);
-    return record_cost(2 * B_H * pairs * D, mfma, !f32 ? 16 : decode ? 32 : 64,
-                       (q.numel() + k.numel() + v.numel()) * es, out.numel() * es);
+    record_cost(2 * B_H * pairs * D, mfma, f32 ? 64 : 16, (q.numel() + k.numel() + v.numel()) * es, out.numel() * es);
+    g_cost->v[KG_COST_MFMA] += split.h16 + split.f32;
+    g_cost->v[KG_COST_MFMA_CYCLES] += 16 * split.h16 + 32 * split.f32;
+    return kOk;
   }
 
   if (decode) {

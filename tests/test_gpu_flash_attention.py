@@ -432,3 +432,34 @@ def test_any_head_dim(device, b, h, s_q, s_kv, d, causal, dtype):
         attention_h16_tolerance(*arrays, scale, causal, dtype)
     assert_within(to_numpy(out), ref, tol, what=f"{(b, h, s_q, s_kv, d)} {causal} {dtype}")
     assert torch.isnan(guard[:256]).all() and torch.isnan(guard[-256:]).all(), "store outside the output"
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("b,h,s_q,s_kv,d,causal", ANY_DIM)
+def test_any_head_dim_keeps_probabilities_in_fp32(device, b, h, s_q, s_kv, d, causal, dtype):
+    """16-bit calls of other head dims round to 16 bits once, in the output: scores, probabilities
+    and both sums are fp32. Reference: the softmax formula in float64 on the rounded inputs. Bar:
+    the output's own rounding (u = 2^-8 for bf16's 8 significand bits, 2^-11 for f16's 11; 2^-25
+    below f16's normal range) of a value that the fp32 arithmetic has moved by at most
+    attention_f32_tolerance's first-order terms (without its flat 1e-5 + 1e-4 |o|, which is
+    no rounding bound). Probabilities in 16 bits miss it where an output cancels: they move O_i by about
+    u sqrt(sum_j w_j^2 (V_j - O_i)^2), which does not shrink with |O_i|."""
+
+    import torch
+
+    tdt = getattr(torch, dtype)
+    rng = np.random.default_rng(3 * s_q + s_kv + d)
+    (q, qn), (k, kn), (v, vn) = (round_to(rng.standard_normal((b, h, s, d), dtype=np.float32), tdt)
+                                 for s in (s_q, s_kv, s_kv))
+    scale = 1.0 / np.sqrt(d)
+    out = torch.full(q.shape, float("nan"), dtype=tdt, device=device)
+    print(f"[fa] fp32 probabilities {(b, h, s_q, s_kv, d)} causal={causal} {dtype}", flush=True)
+    native.flash_attention(out, q.to(device), k.to(device), v.to(device), 64, 64, scale, causal)
+    s = qn.astype(np.float64) @ kn.astype(np.float64).swapaxes(-1, -2) * scale
+    if causal:
+        s = np.where(np.tril(np.ones((s_q, s_kv), bool)), s, -np.inf)
+    w = np.exp(s - s.max(-1, keepdims=True))
+    ref = (w / w.sum(-1, keepdims=True)) @ vn.astype(np.float64)
+    moved = attention_f32_tolerance(qn, kn, vn, scale, causal) - 1e-5 - 1e-4 * np.abs(ref)
+    u = {"bfloat16": 2.0**-8, "float16": 2.0**-11}[dtype]
+    assert_within(to_numpy(out), ref, u * (np.abs(ref) + moved) + 2.0**-25 + moved, what=f"{(b, h, s_q, s_kv, d)} {dtype}")
