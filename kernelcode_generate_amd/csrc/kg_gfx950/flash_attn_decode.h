@@ -35,6 +35,43 @@ constexpr int step_keys() { return D == 128 ? 32 : 64; }  // 16 KiB of K and V
 // The lowest running max: a score of -inf (infinite inputs) has weight 0 beside finite ones,
 // also where a whole step has no other.
 constexpr float kMinMax = -3.0e38f;
+
+// O^T += V^T P^T in fp32 over the 4 NG keys of a step: MFMA n contracts keys key0 + 16 (n/4) +
+// 4 (l/16) + n%4, of which this lane holds query l16's weight p[n] and V's values v(n, e) of block e.
+// masked: the step has keys that some of the queries q0 + 0..15 do not see (their weights are 0). A
+// weight of 0 does not take an infinity or NaN out of the sum, so where such a step holds one,
+// every query gets a pass of its own with zeros in place of the keys after it. Finite values (a test of
+// V's registers in one step per block of queries) take the one pass.
+// non_finite() tests this lane's: on the stored words, as the widened values of a whole step, kept from the
+// test for the products, spilled 256 registers (bf16 16x389x389x80 17 -> 40 us).
+template <int NE, int NG, typename Values, typename Test>
+__device__ __forceinline__ void add_pv_f32(f32x4 (&o)[NE], const float (&p)[NG], Values v, Test non_finite, bool masked,
+                                           int key0, int q0, int l16, int lr) {
+  bool apart = false;
+  if (masked) apart = __builtin_amdgcn_ballot_w64(non_finite()) != 0;
+  if (!apart) {
+#pragma unroll
+    for (int n = 0; n < NG; ++n)
+#pragma unroll
+      for (int e = 0; e < NE; ++e) o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v(n, e), p[n], o[e], 0, 0, 0);
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    f32x4 sum = o[e];
+#pragma unroll 1
+    for (int q = 0; q < kMaxQ; ++q) {
+      f32x4 t = o[e];
+#pragma unroll
+      for (int n = 0; n < NG; ++n) {
+        const float seen = key0 + 16 * (n >> 2) + 4 * lr + (n & 3) <= q0 + q ? v(n, e) : 0.f;
+        t = __builtin_amdgcn_mfma_f32_16x16x4f32(seen, p[n], t, 0, 0, 0);
+      }
+      if (l16 == q) sum = t;
+    }
+    o[e] = sum;
+  }
+}
 }  // namespace fad
 
 // splits == 1: O is written; else partial[(bh splits + split) s_q + q][D + 2] takes O (not
@@ -143,20 +180,26 @@ __global__ __launch_bounds__(fad::kThreads, 2) void fa_decode_kernel(const uint1
       for (int c = 0; c < NE; ++c) o[c] *= alpha;
     }
     if constexpr (kAny) {
-      // P stays fp32 and V's elements are widened: MFMA (kb, i) contracts keys 16kb + 4(l/16) + i
+      // P stays fp32 and V's elements are widened
+      float p[8 * NC];
 #pragma unroll
-      for (int kb = 0; kb < 2 * NC; ++kb)
+      for (int n = 0; n < 8 * NC; ++n) {
+        p[n] = __builtin_amdgcn_exp2f(__builtin_fmaf((float)sc[n >> 2][n & 3], scale_log2, -m_run));
+        l_run[0] += p[n];
+      }
+      auto value = [&](int n, int e) __attribute__((always_inline)) {  // key 16 (n/4) + 4 (l/16) + n%4 of the step
+        const uint32_t pair = b.v[n >> 3][n & 7][e >> 1];
+        return H::to_float((e & 1) ? pair >> 16 : pair & 0xffffu);
+      };
+      auto non_finite = [&]() __attribute__((always_inline)) {  // an exponent of ones carries into its sign bit
+        uint32_t carry = 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf((float)sc[kb][i], scale_log2, -m_run));
-          l_run[0] += p;
-          const VRow row = b.v[kb >> 1][4 * (kb & 1) + i];
+        for (int r = 0; r < 8 * NC; ++r)
 #pragma unroll
-          for (int e = 0; e < NE; ++e) {
-            const uint32_t pair = row[e >> 1];
-            o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(H::to_float((e & 1) ? pair >> 16 : pair & 0xffffu), p, o[e], 0, 0, 0);
-          }
-        }
+          for (int w = 0; w < NE / 2; ++w) carry |= (b.v[r >> 3][r & 7][w] & H::kExpPair) + H::kExpUnitPair;
+        return (carry & 0x80008000u) != 0;
+      };
+      add_pv_f32(o, p, value, non_finite, diagonal && key0 + kStep - 1 > q0, key0, q0, l16, lr);
     } else {
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
@@ -381,10 +424,16 @@ __global__ __launch_bounds__(fad::kThreads, 2) void fa_split_f32_kernel(const fl
       p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf((float)sc[i], scale_log2, -m_run));
       l_run += p[i];
     }
+    auto value = [&](int n, int e) __attribute__((always_inline)) { return b.v[n][e]; };
+    auto non_finite = [&]() __attribute__((always_inline)) {
+      bool any = false;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+      for (int n = 0; n < 4; ++n)
 #pragma unroll
-      for (int e = 0; e < NE; ++e) o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.v[i][e], p[i], o[e], 0, 0, 0);
+        for (int e = 0; e < NE; ++e) any |= !__builtin_isfinite(b.v[n][e]);
+      return any;
+    };
+    add_pv_f32(o, p, value, non_finite, causal != 0 && key0 + kStep - 1 > q0, key0, q0, l16, lr);
   };
 
   constexpr int kStride = kStep * kWaves;

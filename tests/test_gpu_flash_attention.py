@@ -463,3 +463,47 @@ def test_any_head_dim_keeps_probabilities_in_fp32(device, b, h, s_q, s_kv, d, ca
     moved = attention_f32_tolerance(qn, kn, vn, scale, causal) - 1e-5 - 1e-4 * np.abs(ref)
     u = {"bfloat16": 2.0**-8, "float16": 2.0**-11}[dtype]
     assert_within(to_numpy(out), ref, u * (np.abs(ref) + moved) + 2.0**-25 + moved, what=f"{(b, h, s_q, s_kv, d)} {dtype}")
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("b,h,s,d", [(1, 2, 70, 24), (1, 1, 45, 72), (2, 1, 300, 80), (1, 1, 16, 96), (1, 1, 700, 120)])
+def test_causal_masked_values_are_not_read(device, b, h, s, d, dtype):
+    """Head dims of the split-key kernels, causal: an infinity or NaN in V's row j belongs to queries
+    j and later only; earlier queries of the same block keep the bits they have without it. Rows at a
+    block's start, middle and end, one step and several, the last key among them."""
+
+    import torch
+
+    tdt = getattr(torch, dtype)
+    gen = torch.Generator(device=device).manual_seed(s + d)
+    q, k, v = (torch.randn(b, h, s, d, generator=gen, device=device).to(tdt) for _ in range(3))
+    scale = 1.0 / d**0.5
+
+    def run(values):
+        out = torch.full(q.shape, float("nan"), dtype=tdt, device=device)
+        native.flash_attention(out, q, k, values, 64, 64, scale, True)
+        return out
+
+    clean = run(v)
+    assert torch.isfinite(clean).all()
+    for j in sorted({0, 5, 15, s // 2, s // 16 * 16 - 1, s // 16 * 16, s - 1} & set(range(s))):
+        for value in (float("inf"), float("-inf"), float("nan")):
+            print(f"[fa] masked value {value} at key {j} {(b, h, s, d)} {dtype}", flush=True)
+            bad = v.clone()
+            bad[:, :, j, 3] = value
+            bad[:, :, j, d - 1] = value
+            got = run(bad)
+            cols = [3, d - 1]
+            rest = [c for c in range(d) if c not in cols]
+            assert torch.equal(got[:, :, :j], clean[:, :, :j]), f"queries before key {j}"
+            assert torch.equal(got[..., rest], clean[..., rest]), f"other columns, key {j}"
+            seen = got[:, :, j:, cols]
+            # (a weight above fp32's smallest normal: exp(-87); the scores here span far less)
+            assert (torch.isnan(seen) if value != value else seen == value).all(), f"queries from key {j} on"
+
+
+@pytest.mark.parametrize("s,d", [(77, 64), (200, 128)])
+def test_causal_masked_values_are_not_read_small_fp32(device, s, d):
+    """The same for the small fp32 calls with D = 64 and 128 that the split-key kernel takes."""
+
+    test_causal_masked_values_are_not_read(device, 1, 2, s, d, "float32")
