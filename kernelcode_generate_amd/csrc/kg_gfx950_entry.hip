@@ -294,10 +294,10 @@ int pipe_splits(long long M, long long N, long long K, long long* chunk) {
 // the device's pending work (the stream the buffer was used on may no longer exist). Lock
 // order: the table's mutex, then a slot's. An allocation per call (hipMallocAsync /
 // hipFreeAsync) cost about 60 us of host time per matmul.
-// While the stream records a graph there is no workspace: the graph would keep the buffer's
-// address beyond its replacement by any later call on that stream, and allocating invalidates
-// the recording. Every caller then takes its form without one: K or the keys not split, the
-// gathering conv, the SIMT matmul.
+// While a stream records a graph its calls take a buffer of that recording's own, which no other
+// work touches and which lives as long as the graph and its executables (capture_workspace).
+// Every caller also has a form without a workspace, for when there is none to be had: K or the
+// keys not split, the gathering conv, the SIMT matmul.
 constexpr int kSplitCachedStreams = 8;
 struct SplitWorkspace {
   int device;
@@ -314,16 +314,6 @@ struct SplitLease {
 std::mutex g_split_ws_mutex;
 std::vector<SplitWorkspace> g_split_ws;
 unsigned long long g_split_ws_clock = 0;
-
-// True while `stream` records a graph (or cannot be asked because another stream does).
-bool stream_capturing(hipStream_t stream) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
-    (void)hipGetLastError();
-    return true;
-  }
-  return status != hipStreamCaptureStatusNone;
-}
 
 // Allocating is refused, and invalidates the recording, while any other thread records a graph
 // in the global mode, unless the allocating thread is in the relaxed one: its buffers are not
@@ -342,12 +332,110 @@ class RelaxedCaptureMode {
   hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
 };
 
+// Workspaces of recorded graphs: a buffer per recording and stream (the calls of one are in order),
+// shared by that recording's calls that fit it, held by a user object of the graph. The runtime
+// drops it with the last of the graph and its executables; the buffer is then freed by the next
+// call that takes a workspace outside a recording (hipFree, which waits for the device: an
+// executable may be dropped while it runs). At most kCaptureMaxBytes are held in all.
+constexpr size_t kCaptureMaxBytes = 1ull << 30;
+struct CaptureWorkspace {
+  unsigned long long recording;
+  hipStream_t stream;
+  void* ptr;
+  size_t bytes;
+  std::shared_ptr<std::mutex> busy;  // as SplitWorkspace's
+};
+std::vector<CaptureWorkspace> g_capture_ws;  // guarded by g_split_ws_mutex
+// Buffers whose graphs are gone. The runtime may call the destructor with its own locks held and at
+// process exit, so it only appends here, under a lock that no HIP call is made with, and the list
+// is never destroyed.
+struct DroppedBuffers {
+  std::mutex mutex;
+  std::vector<void*> ptrs;
+};
+DroppedBuffers& dropped_buffers() {
+  static DroppedBuffers* list = new DroppedBuffers;
+  return *list;
+}
+void drop_capture_buffer(void* ptr) {
+  DroppedBuffers& list = dropped_buffers();
+  std::lock_guard<std::mutex> lock(list.mutex);
+  list.ptrs.push_back(ptr);
+}
+// (with g_split_ws_mutex held)
+void free_dropped_buffers() {
+  std::vector<void*> ptrs;
+  {
+    DroppedBuffers& list = dropped_buffers();
+    std::lock_guard<std::mutex> lock(list.mutex);
+    ptrs.swap(list.ptrs);
+  }
+  if (ptrs.empty()) return;
+  const RelaxedCaptureMode relaxed;
+  for (void* ptr : ptrs) {
+    (void)hipFree(ptr);
+    g_capture_ws.erase(std::remove_if(g_capture_ws.begin(), g_capture_ws.end(),
+                                      [&](const CaptureWorkspace& w) { return w.ptr == ptr; }),
+                       g_capture_ws.end());
+  }
+}
+// (with g_split_ws_mutex held)
+SplitLease capture_workspace(size_t bytes, hipStream_t stream, unsigned long long recording, hipGraph_t graph) {
+  SplitLease lease;
+  std::shared_ptr<std::mutex> busy;
+  size_t held = 0;
+  for (const auto& w : g_capture_ws) {
+    held += w.bytes;
+    if (w.recording != recording || w.stream != stream) continue;
+    busy = w.busy;
+    if (w.bytes >= bytes) {
+      lease.hold = std::unique_lock<std::mutex>(*busy);
+      lease.ptr = w.ptr;
+      return lease;
+    }
+  }
+  if (held + bytes > kCaptureMaxBytes) return lease;
+  const RelaxedCaptureMode relaxed;
+  void* ptr = nullptr;
+  hipUserObject_t owner = nullptr;
+  if (hipMalloc(&ptr, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return lease;
+  }
+  if (hipUserObjectCreate(&owner, ptr, drop_capture_buffer, 1, hipUserObjectNoDestructorSync) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipFree(ptr);
+    return lease;
+  }
+  if (!busy) busy = std::make_shared<std::mutex>();
+  g_capture_ws.push_back({recording, stream, ptr, bytes, busy});
+  if (hipGraphRetainUserObject(graph, owner, 1, hipGraphUserObjectMove) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipUserObjectRelease(owner, 1);  // drops the buffer
+    return lease;
+  }
+  lease.hold = std::unique_lock<std::mutex>(*busy);
+  lease.ptr = ptr;
+  return lease;
+}
+
 SplitLease split_workspace(size_t bytes, hipStream_t stream) {
   SplitLease lease;
-  if (stream_capturing(stream)) return lease;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long recording = 0;
+  hipGraph_t graph = nullptr;
+  const hipGraphNode_t* dependencies = nullptr;
+  size_t count = 0;
+  if (hipStreamGetCaptureInfo_v2(stream, &status, &recording, &graph, &dependencies, &count) != hipSuccess) {
+    (void)hipGetLastError();  // the null stream, while another one records
+    return lease;
+  }
+  if (status != hipStreamCaptureStatusNone && status != hipStreamCaptureStatusActive) return lease;
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) return lease;
   std::lock_guard<std::mutex> lock(g_split_ws_mutex);
+  if (status == hipStreamCaptureStatusActive) return capture_workspace(bytes, stream, recording, graph);
+  free_dropped_buffers();
   int slot = -1, lru = -1, on_device = 0;
   for (int i = 0; i < (int)g_split_ws.size(); ++i) {
     const auto& w = g_split_ws[i];
@@ -875,8 +963,8 @@ int conv2d_impl(const KgArgSlot* args, unsigned long long n) {
     return finish_launch("conv2d(rowvec)");
   }
   // Everything else: the channel-last copy and its GEMM, or, for tiny calls, a set stage count
-  // (that kernel's ring is its own), without a workspace (while a graph records) and where the
-  // copy does not fit it, the gathering implicit GEMM.
+  // (that kernel's ring is its own), without a workspace and where the copy does not fit it, the
+  // gathering implicit GEMM.
   if (const ConvNhwcPlan plan = conv_nhwc_plan(s, out.dtype == KG_DTYPE_F32, kSplitMaxWorkspace);
       plan.ok && !staged && aligned16(out.data)) {
     lease = split_workspace(plan.bytes(), g_stream);
@@ -1054,7 +1142,7 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
   }
 
   if (decode) {
-    // one range per (b,h) where there is no workspace (while a graph records)
+    // one range per (b,h) where there is no workspace
     FaDecodePlan plan = fa_decode_plan(s, f32, true);
     SplitLease lease;
     if (plan.splits > 1) {
