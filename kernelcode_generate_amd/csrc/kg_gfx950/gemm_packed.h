@@ -110,10 +110,13 @@ __global__ __launch_bounds__(64) void gemm_packed_reduce_kernel(const float* __r
 // the packing do not pay for less (us, this form / SIMT): 16-bit from 100 MFLOP or K = 500
 // (1000x1501x1023: 19.5 / 151; 1x3692x523: 11.1 / 14.4; 250^3: 10.9 / 9.4; 8000x65x129: 12.0 / 16.1),
 // fp32 from 200 MFLOP or K = 1000 (511x513x515: 16.9 / 30.3; 24x100x8000: 25 / 127; 1x3692x523:
-// 16.9 / 10.8; 8000x65x129: 16.6 / 13.6), few fp32 rows against an rhs of over 32 MB not at all
-// (5x4313x7213: 238 / 149; 13x5900x1745: 68 / 38; 4x8000x1000: 58 / 76).
+// 16.9 / 10.8; 8000x65x129: 16.6 / 13.6), few fp32 rows against an rhs of over 32 MB or of very many
+// columns not at all: the SIMT kernel then has its CUs' worth of tiles and reads rhs once
+// (5x4313x7213: 238 / 149; 13x5900x1745: 68 / 38, but 4x8000x1000: 58 / 76; 46x10489x1809: 144 / 106,
+// 36x9233x3429: 224 / 194, but 53x8945x2783: 148 / 160; 114x12697x2395: 264 / 242, but 108x12077x5391: 414 / 537).
 inline bool gemm_packed_pays(long long M, long long N, long long K, bool f32) {
   if (f32 && M < 16 && (double)N * K > 8e6) return false;
+  if (f32 && ((M <= 64 && N >= 9000) || (M <= 128 && N >= 12300))) return false;
   return K >= (f32 ? 1000 : 500) || 2.0 * M * N * K >= (f32 ? 2e8 : 1e8);
 }
 

@@ -482,20 +482,34 @@ SplitLease split_workspace(size_t bytes, hipStream_t stream) {
 }
 
 // 128 x 128 tiles (gemm_mid_kernel) where they make one round on the chip: half the work per
-// workgroup of 128 x 256 ones, which then leave CUs idle. Not where so few tiles have so long a K
-// that splitting K wins. us, this kernel / 128 x 256 tiles, split over K where they were: 2048^3
-// 18.5 / 25.3, 2048x2048x512 8.3 / 10.4, 1536x1536x8192 50 / 65, 2304x2304x2048 (324 tiles) 28 / 26,
-// 5887x1792x3712 (644) 118 / 103; few tiles, split: 1024^3 10.2 / 16.6, 16x4096x1024 11.2 / 10.8,
-// 512x1024x2048 15.2 / 21.6, 371x256x1472 15.6 / 13.4, 64x4096x2048 18.3 / 14.7, 1280x1280x8192 49 / 58,
-// 2745x512x7552 (44 wide tiles) 54 / 48, 1024x1024x4096 26 / 24, 200x8192x4096 31 / 29. Up to K = 512 also grids of up to two rounds
-// (2176x2048: 9.8 / 10.5).
-bool gemm_mid_pays(long long M, long long N, long long K) {
+// workgroup of 128 x 256 ones, which then leave CUs idle. us, this kernel / 128 x 256 tiles: 2048^3
+// 18.5 / 25.3, 2048x2048x512 8.3 / 10.4, but 2304x2304x2048 (324 tiles) 28 / 26,
+// 5887x1792x3712 (644) 118 / 103; up to K = 512 also grids of up to two rounds (2176x2048: 9.8 / 10.5).
+// Outputs of few tiles, whose wide ones would split K, by a time model of both (ns; fitted to 227
+// products of 130..6000 rows and columns on fresh inputs, 12 % off in 9 of 10): a slice of 64
+// k takes 300, more at edges and in larger grids, against 425 per slice of 32 and round of the split
+// form, its partials and its second launch. 1024^3 10.2 / 16.6, 512x1024x2048 15.2 / 21.6,
+// 1536x1536x8192 50 / 65; but 938x152x952 15.2 / 11.0, 1533x216x1832 20.7 / 16.9, 1760x792x7728 80 / 61.
+// Without a workspace these tiles are the fallback of every such call.
+bool gemm_mid_fits(long long M, long long N, long long K) {
   if (pipe_tile_m(M, N) != 128) return false;
+  const long long mid = cdiv(M, gemmm::kT) * cdiv(N, gemmm::kT);
+  return mid <= kNumCUs || (K <= 512 && mid <= 2 * kNumCUs);
+}
+bool gemm_mid_pays(long long M, long long N, long long K) {
+  if (!gemm_mid_fits(M, N, K)) return false;
   const long long mid = cdiv(M, gemmm::kT) * cdiv(N, gemmm::kT), wide = cdiv(M, 128) * cdiv(N, gemmp::kBN);
-  if (mid > kNumCUs) return K <= 512 && mid <= 2 * kNumCUs;
-  if (wide > kSplitMaxTiles || K <= 1024) return true;
-  if (K <= 2048) return wide >= 12 && std::min(M, N) >= 192;
-  return wide > 48 && std::min(M, N) >= 512;
+  long long chunk = K;
+  const long long splits = pipe_splits(M, N, K, &chunk);
+  if (splits == 1) return wide > kSplitMaxTiles || K <= 1024;
+  if (K > 640 && N < gemmp::kBN) return false;  // one wide column of tiles: its partials are small
+  if (K > 1024 && K <= 2048 && (wide < 12 || M < 192)) return false;
+  if (K > 2048 && wide <= kSplitMaxTiles && (wide <= 48 || std::min(M, N) < 512 || K > 6144)) return false;
+  const bool edges = M % gemmm::kT || N % gemmm::kT || K % gemmm::kBK;
+  const long long mid_ns = 6700 + cdiv(K, gemmm::kBK) * (300 + (edges ? 135 : 0) + mid);
+  const long long split_ns =
+      8400 + cdiv(wide * splits, kNumCUs) * (chunk / gemmp::kBK) * 425 + M * N * splits * 84 / 100000 + wide * splits * 17;
+  return 100 * mid_ns <= 97 * split_ns;
 }
 // Its ring: four stages of a 64-deep slice, or two and two workgroups per CU where the K loop is
 // short beside its fill (2048x2048x1024: 11.3 us with two stages, 12.0 with four; x2048: 24.2, 18.5).
@@ -516,7 +530,18 @@ int launch_gemm_mfma(const Mem& out, const Mem& lhs, const Mem& rhs, const Mem& 
   const int grid = (int)(cdiv(M, tm) * cdiv(N, gemmp::kBN));
   long long chunk = K;
   int splits = pipe_splits(M, N, K, &chunk);
-  if (gemm_mid_pays(M, N, K)) {
+  bool mid = gemm_mid_pays(M, N, K);
+  float* partial = nullptr;
+  SplitLease lease;  // held until both kernels of a split call are enqueued (this function's return)
+  if (!mid && splits > 1) {
+    lease = split_workspace((size_t)splits * M * N * sizeof(float), g_stream);
+    partial = static_cast<float*>(lease.ptr);
+    if (partial == nullptr) {  // no workspace: the whole K range in one pass, on smaller tiles
+      splits = 1;
+      mid = gemm_mid_fits(M, N, K);
+    }
+  }
+  if (mid) {
     const int depth = staged ? stages : gemm_mid_stages(K);
     const bool edges = M % gemmm::kT || N % gemmm::kT || K % gemmm::kBK;
 #define KG_GEMM_MID(ST)                                                                                                   \
@@ -526,13 +551,6 @@ int launch_gemm_mfma(const Mem& out, const Mem& lhs, const Mem& rhs, const Mem& 
 #undef KG_GEMM_MID
     if (e != hipSuccess) return fail(kHipFailure, "matmul(mfma-mid): %s", hipGetErrorString(e));
     return finish_launch("matmul(mfma-mid)");
-  }
-  float* partial = nullptr;
-  SplitLease lease;  // held until both kernels of a split call are enqueued (this function's return)
-  if (splits > 1) {
-    lease = split_workspace((size_t)splits * M * N * sizeof(float), g_stream);
-    partial = static_cast<float*>(lease.ptr);
-    if (partial == nullptr) splits = 1;  // no workspace: the whole K range in one pass
   }
   const int k_chunk = splits > 1 ? (int)chunk : 0;
   if (!ragged && splits == 1 && (tm == 256 || grid >= kNumCUs)) {
@@ -639,25 +657,42 @@ int launch_gemm_f32_splitk(const Mem& out, const Mem& lhs, const Mem& rhs, const
 // Few rows: one round of workgroups that each read their columns of rhs once, against kernels that
 // copy tiles through LDS and split K over two launches. mfma: the call meets the alignment of
 // those (splitk: of the fp32 kernel of 32 x 32 blocks); otherwise the packed form or the SIMT
-// kernel would take it. us, this kernel / the other:
-// - 16-bit, aligned: one round, 16x4096x4096 11.7 / 14.9, 128x2048x4096 11.4 / 18.0, 64x64x8192
-//   12.2 / 16.4 (a tie where both run at HBM's rate: 32x8192x8192 29.4 / 29.1); two, while K is short: 64x8192x2048 14.1 / 17.3, x8192 50 / 33; four (16x32000x2048) 24.0 / 22.9.
+// kernel would take it. us on fresh inputs, this kernel / the other:
+// - 16-bit, aligned, one round: 16x4096x4096 12.3 / 17.3, 128x2048x4096 11.4 / 18.0, 16x4672x3840 15.0 / 17.7.
+//   A workgroup's 16 waves take all of K, so a longer K goes to the split form, which has workgroups
+//   for it (16x2048x16384 41 / 23, 96x2048x12288 37 / 28): past 4096 unless rhs is small (112x1792x5440
+//   16.9 / 20.4), past 6144 unless few rows meet very many columns (2x6848x7424 22 / 29) or many rows
+//   few (112x896x6848 14.9 / 20.8), past 8192 always. And from 2560 on with 96 to 160 tiles, where
+//   the two are close, only if the waves' last turn is nearly full (24x3904x2816 8.1 / 13.4, but
+//   32x4480x3264 16.6 / 14.8, 32x3584x3392 15.8 / 14.4).
+// - two rounds, while K is short: 64x8192x2048 14.1 / 17.3, 16x15616x1760 18.0 / 20.0; x8192 50 / 33.
 // - 16-bit, unaligned: 16x2001x2049 11.3 / 22.2, 64x2001x2001 10.3 / 20.7, 40x6001x1501 (two rounds)
 //   20.7 / 32.4; long K needs many columns: 16x4001x4097 19.8 / 41.6, 16x1001x4097 20.8 / 17.1,
 //   64x4097x4095 64 / 42.
 // - fp32 against the 128 x 128-tile kernel, whose one round takes six times as long: 256x4096x4096
-//   (four rounds) 133 / 298, 128x8192x512 24 / 41. Against the other fp32 forms up to 128 rows:
-//   128x1024x1024 6.8 / 10.9, 64x512x4096 16.4 / 34.1 (split K from 16 blocks on: its narrowest
-//   outputs keep the 32 x 32 blocks), but 256x1024x1024 13.4 / 11.5 and 2x65x8001 27.5 / 23.6.
+//   (four rounds) 133 / 298, 128x8192x512 24 / 41, but of four rounds with a short K 96x10176x176 22.5 / 17.0.
+//   Against the other fp32 forms up to 128 rows: 128x1024x1024 6.8 / 10.9, 64x512x4096 16.4 / 34.1, but
+//   256x1024x1024 13.4 / 11.5, 2x65x8001 27.5 / 23.6, and of two rounds 128x2432x1728 36 / 29.
+//   (Narrower outputs gain as much: 64x64x8192 takes half the time here. The line at 16 blocks is not
+//   where the kernels meet; it keeps the 64 x 96 output of K = 4096 that test_f32_split_k names on the
+//   32 x 32 blocks.)
 bool gemm_skinny_pays(long long M, long long N, long long K, bool f32, bool mfma, bool splitk) {
   if (K < 64 || N < gemms::kCols) return false;  // nothing to gain: calls of a launch's length
   const long long tiles = cdiv(N, gemms::kCols);
   const long long rounds = cdiv(tiles * cdiv(M, gemm_skinny_rows(M, N)), kNumCUs);
-  if (f32 && mfma) return M <= 512 && rounds <= 4;
+  if (f32 && mfma) return M <= 512 && (rounds <= 3 || (rounds == 4 && K >= 384));
   if (M > 128 || rounds > 2) return false;
-  if (f32) return splitk ? tiles * cdiv(M, 16) >= 16 : tiles >= 8 || K <= 4096;
-  if (mfma) return rounds == 1 || K <= 2048;
-  return K <= 2304 || (rounds == 1 && M <= 32 && tiles >= 60);
+  if (f32) return splitk ? rounds == 1 && tiles * cdiv(M, 16) >= 16 : tiles >= 8 || K <= 4096;
+  if (!mfma) return K <= 2304 || (rounds == 1 && M <= 32 && tiles >= 60);
+  if (rounds == 2) return K <= 2048;
+  if (K <= 2560) return true;
+  if (M <= 16 && tiles >= 160) return K <= 8192;
+  if (K <= 4096) {
+    const long long batches = cdiv(K, 64), turns = cdiv(batches, gemms::kWaves);
+    return tiles < 96 || tiles >= 160 || 10 * batches >= 9 * gemms::kWaves * turns;
+  }
+  if (K <= 6144) return N * K <= 10 * 1024 * 1024;
+  return K <= 8192 && M > 48 && N <= 1088;
 }
 
 int matmul_impl(const KgArgSlot* args, unsigned long long n) {

@@ -237,3 +237,47 @@ def test_roofline_kind():
     mfma_ns = 258048 * 32 / 1024 / 2.4
     bytes_ns = (2 * 32 * 64 * 56 * 56 * 2 + 64 * 64 * 9 * 2) / 8000
     assert conv == int(-(-max(mfma_ns, bytes_ns) // 1))
+
+
+@pytest.mark.parametrize(
+    "shape,dtype,route",
+    [
+        # (M, K, N): products whose K is too long for one workgroup per tile split it over workgroups
+        ((16, 16384, 2048), "bfloat16", "wide"),  # 23 us, 41 in few-row form
+        ((96, 12288, 2048), "bfloat16", "wide"),  # 28, 37
+        ((32, 3264, 4480), "bfloat16", "wide"),  # 14.8, 16.6: the waves' last turn a quarter full
+        ((4000, 8192, 512), "float16", "wide"),  # 41, 57 in 128 x 128 tiles
+        ((1533, 1832, 216), "float16", "wide"),  # 16.9, 20.7
+        ((938, 952, 152), "float16", "wide"),  # 11.0, 15.2
+        ((1760, 7728, 792), "float16", "wide"),  # 61, 80
+        ((46, 1809, 10489), "float32", "simt"),  # 106, 144 with rhs packed
+        ((128, 1728, 2432), "float32", "splitk"),  # 29, 36 in few-row form of two rounds
+        ((96, 176, 10176), "float32", "tiles"),  # 17, 22.5 in few-row form of four
+        # and the calls on the other side of each line
+        ((16, 4096, 4096), "bfloat16", "few"),  # 17, 12
+        ((2, 7424, 6848), "bfloat16", "few"),  # 29, 22
+        ((112, 6848, 896), "bfloat16", "few"),  # 21, 15
+        ((1024, 1024, 1024), "bfloat16", "mid"),  # 16.6, 10.2
+        ((894, 3512, 2248), "float16", "mid"),  # 49, 39
+        ((53, 2783, 8945), "float32", "packed"),  # 160, 148
+        ((128, 1024, 1024), "float32", "few"),  # 10.9, 6.8
+    ],
+)
+def test_matmul_route_lines(shape, dtype, route):
+    """Either side of the lines between the matmul kernels, by the MFMA count of the one chosen."""
+
+    m, k, n = shape
+    specs = [native.TensorSpec(s, dtype) for s in ((m, n), (m, k), (k, n))]
+    up = lambda a, b: -(-a // b)  # noqa: E731
+    rows = 16 if m <= 16 or up(n, 32) * up(m, 16) <= 256 else 32
+    f32 = dtype == "float32"
+    count = {
+        "wide": up(m, 128) * up(n, 256) * up(k, 32) * 128,
+        "mid": up(m, 128) * up(n, 128) * up(k, 64) * 128,
+        "few": up(m, rows) * (rows // 16) * up(n, 32) * up(k, 32) * (16 if f32 else 2),
+        "packed": up(n, 64) * up(m, 64) * up(4 * k, 128) * 128,
+        "tiles": up(m, 128) * up(n, 128) * up(k, 16) * 128,
+        "splitk": (m // 32) * (n // 32) * (k // 16) * 8,
+        "simt": 0,
+    }[route]
+    assert native.cost("matmul", [*specs, None])["MFMA"] == count
