@@ -246,9 +246,8 @@ def test_roofline_kind():
         ((16, 16384, 2048), "bfloat16", "wide"),  # 23 us, 41 in few-row form
         ((96, 12288, 2048), "bfloat16", "wide"),  # 28, 37
         ((32, 3264, 4480), "bfloat16", "wide"),  # 14.8, 16.6: the waves' last turn a quarter full
-        ((4000, 8192, 512), "float16", "wide"),  # 41, 57 in 128 x 128 tiles
-        ((1533, 1832, 216), "float16", "wide"),  # 16.9, 20.7
-        ((938, 952, 152), "float16", "wide"),  # 11.0, 15.2
+        ((2560, 8128, 640), "float16", "wide"),  # 63, 72 in 128 x 128 tiles
+        ((1024, 2048, 328), "float16", "wide"),  # 15.9, 18.8
         ((1760, 7728, 792), "float16", "wide"),  # 61, 80
         ((46, 1809, 10489), "float32", "simt"),  # 106, 144 with rhs packed
         ((128, 1728, 2432), "float32", "splitk"),  # 29, 36 in few-row form of two rounds
