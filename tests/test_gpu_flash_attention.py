@@ -359,8 +359,8 @@ def test_few_queries(device, b, h, s_q, s_kv, d, dtype):
 
 
 def test_few_queries_under_capture(device):
-    """While a graph records, the keys of a (b,h) are not split (no workspace); every replay
-    gives the softmax formula's result."""
+    """A graph's call with split keys has a workspace of the graph's own; every replay gives the
+    softmax formula's result."""
 
     import torch
 

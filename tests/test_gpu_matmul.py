@@ -197,16 +197,23 @@ def test_four_wave_128_row_tiles_match_eight_wave_kernel(device, dtype_name, bia
         assert torch.equal(full[r0:r0 + 1000], part), f"rows {r0}:{r0 + 1000}"
 
 
+def wide_tile_mfma(m, k, n):
+    """MFMA instructions in 128 x 256 tiles; no shape below has as many in 128 x 128 ones or in few-row
+    form, so a cost record equal to it shows the route (K is split by the shape alone then)."""
+
+    return -(-m // 128) * -(-n // 256) * -(-k // 32) * 128
+
+
 @pytest.mark.parametrize(
     "shape,dtype_name,bias_kind,rows",
     [
-        ((16, 4096, 4096), "bfloat16", "f32", None),  # 16 tiles: 16 K chunks of 256
-        ((128, 8192, 1024), "float16", "same", [(0, 16), (112, 128)]),  # 4 tiles: 32 chunks
-        ((3, 1000, 136), "bfloat16", "none", None),  # one ragged tile, last chunk 8 deep short of a slice
-        ((40, 2048, 520), "float16", "f32", None),  # 3 tiles, ragged N
-        ((2048, 4096, 2048), "bfloat16", "f32", [(0, 16), (2032, 2048)]),  # 128 tiles, long K: 2 chunks
+        ((371, 1472, 328), "bfloat16", "f32", None),  # 6 tiles: 5 K chunks
+        ((16, 16384, 2088), "bfloat16", "none", None),  # 9 tiles of few rows, long K: 29 chunks
+        ((136, 1000, 136), "bfloat16", "none", None),  # 2 ragged tiles, last chunk 24 deep short of a slice's end
+        ((300, 2048, 520), "float16", "f32", None),  # 9 tiles, ragged M and N
+        ((2000, 4104, 520), "float16", "same", [(0, 16), (1984, 2000)]),  # 48 tiles, long K: 6 chunks
     ],
-    ids=["16x4096x4096", "128x8192x1024", "3x1000x136", "40x2048x520", "2048x4096x2048"],
+    ids=["371x1472x328", "16x16384x2088", "136x1000x136", "300x2048x520", "2000x4104x520"],
 )
 def test_split_k_skinny(device, oracle_mod, shape, dtype_name, bias_kind, rows):
     """Outputs of few tiles run the pipelined kernel split over K (fp32 partial sums in a
@@ -228,6 +235,8 @@ def test_split_k_skinny(device, oracle_mod, shape, dtype_name, bias_kind, rows):
         bt, bias = round_to(rng.standard_normal(n), dt)
     big = torch.full((m + 2, n + 8), float("nan"), dtype=dt, device=device)
     out = big[:m, :n]
+    specs = [native.TensorSpec.of(out), *(native.TensorSpec(x, dtype_name) for x in ((m, k), (k, n)))]
+    assert native.cost("matmul", [*specs, None])["MFMA"] == wide_tile_mfma(m, k, n)
     print(f"[matmul] split-K M={m} K={k} N={n} {dtype_name} bias={bias_kind}", flush=True)
     native.matmul(out, lt.to(device), rt.to(device), None if bt is None else torch.as_tensor(bt).to(device))
     got = to_numpy(big)
@@ -249,7 +258,9 @@ def test_split_k_on_many_streams(device, oracle_mod):
 
     import torch
 
-    m, k, n = 16, 2048, 512  # 2 output tiles, K split 8 ways
+    m, k, n = 136, 2048, 328  # 4 output tiles, K split 8 ways
+    specs = [native.TensorSpec(x, "bfloat16") for x in ((m, n), (m, k), (k, n))]
+    assert native.cost("matmul", [*specs, None])["MFMA"] == wide_tile_mfma(m, k, n)
     streams = [torch.cuda.Stream(device=device) for _ in range(11)]
     cases = []
     for rnd in range(2):
@@ -472,9 +483,9 @@ def test_memory_stage_depths_bit_identical(device, oracle_mod, shape):
 @pytest.mark.parametrize(
     "shape,bias_kind,strided",
     [
-        ((65, 1001, 129), "same", False),  # one column past a tile, K one past a chunk
+        ((193, 1001, 129), "same", False),  # one row and column past a tile, K one past a chunk
         ((301, 1001, 97), "f32", True),  # odd row strides and bases
-        ((1, 2003, 333), "none", False),  # one row, K split
+        ((1, 4103, 199), "none", False),  # one row, K split
         ((130, 1000, 1003), "same", False),  # lhs aligned, rhs and out not
         ((520, 1015, 520), "f32", True),  # K % 8 = 7: whole 8-column store pieces
         ((3000, 1001, 1501), "none", False),  # 128-column tiles
@@ -508,8 +519,9 @@ def test_unaligned_rows_on_matrix_cores(device, shape, bias_kind, strided, dtype
     big = torch.full((m + 2, n + (8 if n % 8 == 0 else 3)), float("nan"), dtype=dt, device=device)
     out = big[:m, :n]
     spec = [native.TensorSpec.of(t) if t is not None else None for t in (out, a, b, bias)]
-    model = native.cost("matmul", spec)
-    assert model["MFMA"] > 0 and model["MFMA_CYCLES"] == model["MFMA"] * (32 if dt == torch.float32 else 16)
+    # 64 x 64 tiles (two make a 128-column one) of 128-byte slices; no few-row call has as many MFMAs
+    tiles, slices = -(-n // 64) * -(-m // 64), -(-k * a.element_size() // 128)
+    assert native.cost("matmul", spec)["MFMA"] == tiles * slices * (128 if dt == torch.float32 else 32)
     print(f"[matmul] packed {dtype_name} M={m} K={k} N={n} lda={a.stride(0)} ldb={b.stride(0)} ldc={out.stride(0)}", flush=True)
     native.matmul(out, a, b, bias)
     ref = a.double() @ b.double()
@@ -525,14 +537,16 @@ def test_unaligned_rows_on_matrix_cores(device, shape, bias_kind, strided, dtype
 
 
 def test_unaligned_rows_under_capture(device):
-    """While a graph records, the packed form's workspace is not used: the call keeps the SIMT
-    kernel, and every replay gives its bits."""
+    """A graph's packed call has a workspace of the graph's own: every replay gives the bits of the
+    call outside it, whose workspace is another."""
 
     import torch
 
-    a = torch.randn(70, 1001, device=device).half()
+    a = torch.randn(170, 1001, device=device).half()
     b = torch.randn(1001, 99, device=device).half()
-    out = torch.empty(70, 99, dtype=torch.float16, device=device)
+    out = torch.empty(170, 99, dtype=torch.float16, device=device)
+    specs = [native.TensorSpec.of(x) for x in (out, a, b)]
+    assert native.cost("matmul", [*specs, None])["MFMA"] == 2 * 3 * 16 * 32  # packed: 64 x 64 tiles, 16 slices
     stream = torch.cuda.Stream(device=device)
     stream.wait_stream(torch.cuda.current_stream())
     graph = torch.cuda.CUDAGraph()
@@ -551,7 +565,7 @@ def test_unaligned_rows_under_capture(device):
         torch.cuda.synchronize()
         assert ((out.double() - ref).abs() <= tol).all()
         native.matmul(eager, a, b, None)
-        assert ((eager.double() - ref).abs() <= tol).all()
+        assert torch.equal(eager, out)
 
 
 @pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
@@ -608,13 +622,14 @@ def test_128_tiles_match_wide_tiles(device, shape, bias_kind, dtype_name):
         ((3, 65, 33), "same", True),  # one k past a batch, one column past a tile
         ((17, 1023, 95), "f32", True),  # one row past a block; the last step one short, odd N
         ((33, 1089, 2049), "same", True),  # K one past 17 batches, the last pair shifted
-        ((64, 2112, 8200), "none", False),  # 32-row blocks, 257 tiles, one batch per wave and a second
+        ((64, 2048, 8192), "none", False),  # 32-row blocks, two rounds of them, two batches per wave
         ((128, 1120, 999), "same", True),  # 16-row blocks, K half a batch over
-        ((100, 160, 4100), "f32", True),  # 32-row blocks of a ragged M
+        ((100, 160, 4000), "f32", True),  # 32-row blocks of a ragged M, two and a half batches
+        ((40, 1501, 6001), "same", True),  # 32-row blocks, the last of 8 rows; K one short of a slice past 23 batches
     ],
 )
 def test_few_rows(device, shape, bias_kind, odd, dtype_name):
-    """The few-row kernel against float64: an output is rounded once (bf16 2^-9, f16 2^-12 of it, fp32
+    """The few-row kernel (by the cost record, for each type) against float64: an output is rounded once (bf16 2^-9, f16 2^-12 of it, fp32
     covered by the sums) and its products are summed in fp32 in any order: at most k roundings of
     2^-24 of sum |a b|. odd: operands and output are windows of wider buffers with odd row strides and bases;
     nothing outside the output window is written. Rows of k past the end hold NaN."""
@@ -635,6 +650,10 @@ def test_few_rows(device, shape, bias_kind, odd, dtype_name):
         bias = bias.to(dt)
     wide = torch.full((m + 1, n + 2 * pad), float("nan"), dtype=dt, device=device)
     out = wide[:m, pad : pad + n]
+    rows = 16 if m <= 16 or -(-n // 32) * -(-m // 16) <= 256 else 32
+    specs = [native.TensorSpec.of(t) for t in (out, a, b)]
+    blocks = -(-m // rows) * (rows // 16) * -(-n // 32) * -(-k // 32)
+    assert native.cost("matmul", [*specs, None])["MFMA"] == blocks * (16 if dt == torch.float32 else 2)
     print(f"[matmul] few rows {shape} {dtype_name}", flush=True)
     native.matmul(out, a, b, bias)
     ref, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
@@ -651,8 +670,8 @@ def test_few_rows(device, shape, bias_kind, odd, dtype_name):
 
 @pytest.mark.parametrize("shape", [(5, 700, 333), (170, 1001, 99)], ids=["fewrows", "packed"])
 def test_matmul_under_capture(device, shape):
-    """A graph holds a few-row call (one launch, no workspace) and one whose packed form gives way to
-    the SIMT kernel; each replay reads its inputs anew."""
+    """A graph holds a few-row call (one launch, no workspace) or a packed one (a workspace of the
+    graph's own); each replay reads its inputs anew."""
 
     import torch
 

@@ -87,17 +87,20 @@ def test_sync_and_stream_threads(device, oracle_mod):
 def test_split_k_threads_on_one_stream(device, oracle_mod):
     """Two synchronous threads on the one default stream, both running split-K matmuls
     (two kernels per call: fp32 partials in the per-stream workspace, then their ordered
-    reduction) of different sizes, so the workspace is also replaced while the other thread
-    uses it. Each call must hold the workspace from its partials through its reduction:
+    reduction) of different sizes (tests/test_gpu_workspace.py: the other calls that take one, and
+    its replacement meanwhile). Each call must hold the workspace from its partials through its reduction:
     every result equals the single-threaded one bit for bit (the split is deterministic)."""
 
     import torch
 
     rng = np.random.default_rng(7)
-    shapes = ((16, 4096, 4096), (64, 1024, 8192))  # 16 and 4 output tiles: 16- and 32-way K splits
+    shapes = ((371, 328, 1472), (384, 1064, 2560))  # 6 and 15 output tiles: 5- and 10-way K splits
     operands, expected = [], []
     native.set_launch_mode(True, None)
     for m, n, k in shapes:
+        specs = [native.TensorSpec(x, "bfloat16") for x in ((m, n), (m, k), (k, n))]
+        # 128 x 256 tiles in 32-deep slices (other tilings of these shapes issue other counts)
+        assert native.cost("matmul", [*specs, None])["MFMA"] == -(-m // 128) * -(-n // 256) * -(-k // 32) * 128
         a = round_to(rng.standard_normal((m, k), dtype=np.float32) * 0.05, torch.bfloat16)[0].to(device)
         b = round_to(rng.standard_normal((k, n), dtype=np.float32) * 0.05, torch.bfloat16)[0].to(device)
         out = torch.empty((m, n), dtype=torch.bfloat16, device=device)
@@ -105,7 +108,7 @@ def test_split_k_threads_on_one_stream(device, oracle_mod):
         operands.append((a, b))
         expected.append(out.clone())
     ref = oracle_mod.matmul_demo(to_numpy(operands[0][0]), to_numpy(operands[0][1]), None, (64, 64, 64))
-    assert_h16_close(to_numpy(expected[0]), ref, "split-K 16x4096x4096")
+    assert_h16_close(to_numpy(expected[0]), ref, "split-K 371x328x1472")
     torch.cuda.synchronize()
     rounds = 30
     errors: list[BaseException] = []

@@ -17,10 +17,10 @@ pytestmark = pytest.mark.gpu
 
 # name: (operation, dtype, sizes, MFMA instructions of the route meant)
 CALLS = {
-    # matmul (M, K, N): 3 tiles of 128 x 256 and 46 slices of 32, in 5 K chunks
-    "matmul_split": ("matmul", "bfloat16", (371, 1472, 256), 3 * 46 * 128),
-    # 12 tiles of 128 x 256 and 80 slices, in 10 chunks (15.7 MB of partials)
-    "matmul_split_large": ("matmul", "bfloat16", (384, 2560, 1024), 12 * 80 * 128),
+    # matmul (M, K, N): 6 tiles of 128 x 256 and 46 slices of 32, in 5 K chunks
+    "matmul_split": ("matmul", "bfloat16", (371, 1472, 328), 6 * 46 * 128),
+    # 15 tiles of 128 x 256 and 80 slices, in 10 chunks (16.3 MB of partials)
+    "matmul_split_large": ("matmul", "bfloat16", (384, 2560, 1064), 15 * 80 * 128),
     # odd rows: 6 tiles of 64 x 64 and 63 slices of 64, in 7 chunks
     "matmul_packed": ("matmul", "float16", (170, 4001, 99), 6 * 63 * 32),
     "matmul_packed_f32": ("matmul", "float32", (170, 4001, 99), 6 * 126 * 128),
