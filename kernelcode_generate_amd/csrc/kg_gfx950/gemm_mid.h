@@ -63,7 +63,7 @@ __global__ __launch_bounds__(gemmm::kThreads, kStages == 2 ? 2 : 1) void gemm_mi
   // rows depends on the lane and p's parity. rhs piece p: k-rows (wave*4 + p)*4 + lane/16, slot
   // lane%16; b_mask depends on the lane and p/2 ----
   uint32_t a_off[4], b_off[4];
-  int a_k[2], b_col[2];  // a lane's k within the slice (by parity), its column (by p/2)
+  int a_k[2];  // a lane's k within the slice, by p's parity
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
     const int row = (wave * 4 + p) * 8 + (lane >> 3);
@@ -74,7 +74,6 @@ __global__ __launch_bounds__(gemmm::kThreads, kStages == 2 ? 2 : 1) void gemm_mi
     const int k = (wave * 4 + p) * 4 + (lane >> 4);
     const int bc = 8 * ((lane & 15) ^ b_mask(k));
     b_off[p] = (uint32_t)((k * ldb + bc) * 2);
-    b_col[p >> 1] = bc;
     if (kRagged && n0 + bc >= N) b_off[p] = kBufOOB;
   }
   const char* a_tile = reinterpret_cast<const char*>(A + (long long)m0 * lda);

@@ -1126,11 +1126,11 @@ int flash_attention_impl(const KgArgSlot* args, unsigned long long n) {
   if (g_cost == nullptr && out.numel() == 0) return finish_launch("flash_attention(empty)");
   if (s.d > 512) return fail(kUnsupported, "flash_attention: head dim %d > 512", s.d);
   if (s.causal && s.s_kv != s.s_q) return fail(kUnsupported, "flash_attention: causal mask needs S_q == S_kv");
-  // few queries, or a head dim of its own: keys split over workgroups (a call that sets a ring depth takes the kernel with
-  // the ring)
+  // few queries, a head dim of its own or a small fp32 call: keys split over workgroups (a call that
+  // sets a ring depth takes the kernel with the ring)
   const bool f32 = out.dtype == KG_DTYPE_F32;
-  const bool decode = !staged && out.numel() > 0 && fa_split_supported(s, f32) && aligned16(q.data) && aligned16(k.data) && aligned16(v.data) &&
-                      aligned16(out.data);
+  const bool decode = !staged && out.numel() > 0 && fa_split_supported(s, f32) && aligned16(q.data) &&
+                      aligned16(k.data) && aligned16(v.data) && aligned16(out.data);
   if (g_cost) {
     const long long B_H = (long long)s.bh, D = s.d;
     // products Q.K^T and P.V that the mask keeps: causal row i sees keys 0..i

@@ -28,7 +28,7 @@ def out_hw(xs, ws, stride, dil, pad):
     return ho, wo
 
 
-def run(device, dtype, x, w, bias, stride, dil, pad, tiles=()):
+def run(device, dtype, x, w, bias, stride, dil, pad, tiles=(), memory_stage=None):
     import torch
 
     xt = torch.as_tensor(x).to(device)
@@ -37,7 +37,7 @@ def run(device, dtype, x, w, bias, stride, dil, pad, tiles=()):
     ho, wo = out_hw(xt.shape, wt.shape, stride, dil, pad)
     out = torch.full((xt.shape[0], wt.shape[0], ho, wo), float("nan"), dtype=dtype, device=device)
     print(f"[conv2d] x={tuple(xt.shape)} w={tuple(wt.shape)} s={stride} d={dil} p={pad} {dtype}", flush=True)
-    native.conv2d(out, xt, wt, bt, stride, dil, pad, tiles)
+    native.conv2d(out, xt, wt, bt, stride, dil, pad, tiles, memory_stage)
     return out
 
 
@@ -127,7 +127,9 @@ def test_general_params_f32(device, oracle_mod, xs, ws, stride, dil, pad):
 )
 def test_implicit_gemm_shapes(device, oracle_mod, dtype_name, xs, ws, stride, dil, pad, bias):
     """Every conv the 3x3 kernel does not take runs as an implicit GEMM on matrix cores (16-bit
-    or fp32 MFMA); grids of fewer than two workgroups per CU split K into fp32 partials added in
+    or fp32 MFMA): by default over a channel-last copy or on row pieces or, where neither pays, with
+    gathered operands; with a stage count set on row pieces or gathered. Grids of fewer than two
+    workgroups per CU split K into fp32 partials added in
     a fixed order (the 1x1, ragged, dilated and the last two cases). Reference: the oracle's
     demo loop nest on the identically rounded inputs.
     fp32 tolerance: the demo's rtol 1e-4 / atol 1e-5 plus the rounding that two fp32 summation
@@ -157,15 +159,16 @@ def test_implicit_gemm_shapes(device, oracle_mod, dtype_name, xs, ws, stride, di
             bt, b = round_to(rng.normal(size=(ws[0],)).astype(np.float32), dt)
     tiles = (16, 16, 1, 8, 16)
     ref = oracle_mod.conv2d_demo(x, w, b, stride, dil, pad, tiles)
-    out = to_numpy(run(device, dt, xt, wt, bt, stride, dil, pad))
-    what = f"{dtype_name} {xs} {ws} s={stride} d={dil} p={pad} bias={bias}"
-    if dt == torch.float32:
-        terms = oracle_mod.conv2d_demo(np.abs(x), np.abs(w), None, stride, dil, pad, tiles).astype(np.float64)
-        tol = 1e-4 * np.abs(ref) + 1e-5 + 4 * np.sqrt(k) * 2.0 ** -24 * terms
-        err = np.abs(out.astype(np.float64) - ref)
-        assert (err <= tol).all(), f"{what}: max err/tol {np.max(err / tol):.3g}"
-    else:
-        assert_h16_close(out, ref, what=what)
+    for stage in (None, 2):
+        out = to_numpy(run(device, dt, xt, wt, bt, stride, dil, pad, memory_stage=stage))
+        what = f"{dtype_name} {xs} {ws} s={stride} d={dil} p={pad} bias={bias} stage={stage}"
+        if dt == torch.float32:
+            terms = oracle_mod.conv2d_demo(np.abs(x), np.abs(w), None, stride, dil, pad, tiles).astype(np.float64)
+            tol = 1e-4 * np.abs(ref) + 1e-5 + 4 * np.sqrt(k) * 2.0 ** -24 * terms
+            err = np.abs(out.astype(np.float64) - ref)
+            assert (err <= tol).all(), f"{what}: max err/tol {np.max(err / tol):.3g}"
+        else:
+            assert_h16_close(out, ref, what=what)
 
 
 @pytest.mark.parametrize("dtype_name", ["float16", "bfloat16"])

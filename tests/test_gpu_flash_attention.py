@@ -91,17 +91,27 @@ def test_extensions_f32(device, oracle_mod, scale, causal):
         ((1, 1, 1000, 64), 1000, True),
         ((1, 2, 1, 128), 1, False),  # one query, one key
         ((1, 1, 33, 64), 1000, False),
+        ((1, 40, 256, 128), 256, False),  # more than 512 blocks of 16 queries from here on
+        ((2, 20, 230, 128), 230, True),  # partial query block and key tail, causal
+        ((8, 16, 65, 64), 300, False),
+        ((1, 33, 250, 64), 250, True),
     ],
 )
 def test_f32_matrix_cores(device, oracle_mod, shape, s_kv, causal):
-    """fp32 Q/K/V with D in {64, 128} take the fp32 MFMA kernel; the oracle's demo loop nest
-    is the reference where S_q == S_kv, the float64 closed form of the demo's check
-    (kernel/flash_attention/inputs_static_tile_static.py:57-87) otherwise."""
+    """fp32 Q/K/V with D in {64, 128} take an fp32 MFMA kernel: the tiled one (32x32x2 MFMAs of 64
+    cycles), or up to 512 blocks of 16 queries the split-key one (16x16x4, 32 cycles), as the
+    cost record tells. The oracle's demo loop nest is the reference where S_q == S_kv, the float64
+    closed form of the demo's check (kernel/flash_attention/inputs_static_tile_static.py:57-87)
+    otherwise."""
 
     import torch
 
     b, h, sq, d = shape
     scale = 1.0 / np.sqrt(d)
+    specs = [native.TensorSpec(x, "float32") for x in (shape, shape, (b, h, s_kv, d), (b, h, s_kv, d))]
+    model = native.cost("flash_attention", [*specs, 64, 64, scale, int(causal)])
+    cycles = 32 if sq <= 16 or b * h * -(-sq // 16) <= 512 else 64
+    assert model["MFMA"] > 0 and model["MFMA_CYCLES"] == cycles * model["MFMA"]
     rng = np.random.default_rng(sq * 3 + s_kv + d)
     q = rng.standard_normal(shape, dtype=np.float32)
     k, v = (rng.standard_normal((b, h, s_kv, d), dtype=np.float32) for _ in range(2))

@@ -291,12 +291,13 @@ def test_split_k_on_many_streams(device, oracle_mod):
         ((4224, 40, 4104), None),  # 256-row tiles, half a last tile row, 8 columns over, K = 40
         ((520, 4096, 776), None),  # 128-row tiles, long K
         ((4000, 4000, 4000), [(0, 32), (3968, 4000)]),  # 256-row tiles, ragged M and N
+        ((2100, 1000, 2312), [(0, 32), (2068, 2100)]),  # 170 tiles of 128 x 256, more than a round of 128 x 128
     ],
-    ids=["1000x520x1000", "4224x40x4104", "520x4096x776", "4000^3"],
+    ids=["1000x520x1000", "4224x40x4104", "520x4096x776", "4000^3", "2100x1000x2312"],
 )
 def test_ragged_edges_store_only_inside(device, oracle_mod, shape, rows):
-    """Shapes that are not tile multiples take the pipelined kernel's ragged mode: edge copies
-    land zeros and the epilogue masks its stores. The output is a window of a NaN-filled
+    """Shapes that are not tile multiples take the ragged mode of the pipelined kernel or of the one of
+    128 x 128 tiles: edge copies land zeros and the epilogue masks its stores. The output is a window of a NaN-filled
     buffer with 3 extra rows and 8 extra columns, which must stay NaN."""
 
     import torch
