@@ -18,13 +18,17 @@
  * "runtime_throw_or_abort") is unchanged.
  *
  * Memory slots carry DEVICE pointers (torch ROCm tensor .data_ptr()), element shapes
- * and element strides. Kernels allocate nothing per call, with one exception: matmul and
- * conv2d calls that split K over workgroups keep their fp32 partial sums in a workspace
- * held per (device, stream) for the life of the process, allocated on the first such call
- * on that stream and reallocated when a later one needs more. Those calls are therefore
- * not safe under HIP graph capture unless an earlier call of at least the same size ran on
- * that stream uncaptured. Calls are synchronous by default (the reference's cuda_sm89
- * launch ends with a device synchronize, include/cuda_sm89/Arch.h:166-168);
+ * and element strides. Kernels allocate nothing per call, with one exception: calls that need
+ * memory between their launches (fp32 partial sums of a K split over workgroups, packed operands
+ * of matmuls with unaligned rows, a conv's channel-last copy, partial outputs of split attention
+ * keys) take it from a workspace held per (device, stream) for the life of the process (at most
+ * 64 MiB, for 8 streams per device), allocated on the first such call on that stream and
+ * reallocated when a later one needs more. While a stream records a HIP graph such calls take a
+ * buffer that belongs to the graph instead: it is allocated during the recording, lives as long as
+ * the graph and its executables, and is freed by a later call that takes a workspace outside a
+ * recording (at most 1 GiB of such buffers; beyond it calls take forms that need none).
+ * Calls are synchronous by default (the reference's cuda_sm89 launch ends with a device
+ * synchronize, include/cuda_sm89/Arch.h:166-168);
  * kg_gfx950_set_launch_mode() switches to asynchronous launches on a caller-chosen stream
  * for benchmarking.
  *
@@ -83,7 +87,8 @@ typedef struct KgArgSlot {
  * kernel_gen/passes/memory/multi_buffer.py; default 4); other kernels ignore it.
  * 16-bit outputs of at most 64 tiles of 128 x 256 with K >= 512 split K over workgroups and
  * add the fp32 partial sums in a second kernel; the partials live in a workspace the library
- * allocates once per (device, stream) on first use (hipMalloc, at most 64 MiB) and keeps.
+ * allocates once per (device, stream) on first use (hipMalloc, at most 64 MiB) and keeps
+ * (recorded graphs: see the top of this file). Rows of any alignment are packed into it first.
  */
 int kg_gfx950_matmul_entry(const KgArgSlot* ordered_args, unsigned long long arg_count);
 
@@ -98,7 +103,8 @@ int kg_gfx950_matmul_entry(const KgArgSlot* ordered_args, unsigned long long arg
  * which forwards the constants here. Ho/Wo follow kernel/conv2d/inputs_static_tile_static.py:155-156.
  * 16-bit and fp32 convs whose grid would leave CUs idle (small batches, deep 14x14 / 7x7
  * layers) split the contraction over workgroups and add the fp32 partial sums in a second
- * kernel, in the matmul's per-(device, stream) workspace (allocated on first use, kept).
+ * kernel, in the matmul's per-(device, stream) workspace (allocated on first use, kept); most
+ * convs outside the row-piece kernels write a channel-last copy of their image there first.
  */
 int kg_gfx950_conv2d_entry(const KgArgSlot* ordered_args, unsigned long long arg_count);
 
@@ -109,7 +115,8 @@ int kg_gfx950_conv2d_entry(const KgArgSlot* ordered_args, unsigned long long arg
  *   (out[B,H,S,D], q[B,H,S,D], k[B,H,S,D], v[B,H,S,D] [, br, bc [, scale, causal]])
  * 4, 6 or 8 slots. The reference computes softmax(Q K^T) V with no scale and no mask;
  * slots 6-7 are an additive extension: FLOAT scale (default 1.0) and INT causal
- * (0/1, lower-triangular mask including the diagonal).
+ * (0/1, lower-triangular mask including the diagonal). Calls of few queries, or of few blocks of
+ * queries, split their keys over workgroups, with partial outputs in the same workspace.
  */
 int kg_gfx950_flash_attention_entry(const KgArgSlot* ordered_args, unsigned long long arg_count);
 
