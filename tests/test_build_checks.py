@@ -28,6 +28,7 @@ from pathlib import Path
 import pytest
 
 from kernelcode_generate_amd import native
+from kernelcode_generate_amd.build import SOURCES
 
 LLVM = Path("/opt/rocm/llvm/bin")
 TARGET = "hipv4-amdgcn-amd-amdhsa--gfx950"
@@ -41,18 +42,24 @@ def _disassemble(tmp_path: Path) -> list[str]:
     if not all(t.exists() for t in tools):
         pytest.skip("ROCm LLVM tools are not installed")
     fat = tmp_path / "fat.bin"
-    co = tmp_path / "gfx950.co"
     subprocess.run([str(tools[0]), f"--dump-section=.hip_fatbin={fat}", str(lib), str(tmp_path / "host.o")],
                    check=True, capture_output=True)
-    subprocess.run([str(tools[1]), "--unbundle", "--type=o", f"--targets={TARGET}", f"--input={fat}",
-                    f"--output={co}"], check=True, capture_output=True)
-    out = subprocess.run([str(tools[2]), "-d", "--mcpu=gfx950", str(co)], check=True, capture_output=True,
-                         text=True).stdout
+    # one bundle per translation unit, one after another
+    data, magic = fat.read_bytes(), b"__CLANG_OFFLOAD_BUNDLE__"
+    starts = [m.start() for m in re.finditer(magic, data)]
+    assert len(starts) == len(SOURCES)
     lines = []
-    for line in out.splitlines():
-        text = line.split("//", 1)[0].strip()
-        if text and not text.endswith(">:") and not text.startswith("Disassembly") and ":" not in text.split()[0]:
-            lines.append(text)
+    for n, (start, end) in enumerate(zip(starts, [*starts[1:], len(data)])):
+        part, co = tmp_path / f"part{n}.bin", tmp_path / f"gfx950_{n}.co"
+        part.write_bytes(data[start:end])
+        subprocess.run([str(tools[1]), "--unbundle", "--type=o", f"--targets={TARGET}", f"--input={part}",
+                        f"--output={co}"], check=True, capture_output=True)
+        out = subprocess.run([str(tools[2]), "-d", "--mcpu=gfx950", str(co)], check=True, capture_output=True,
+                             text=True).stdout
+        for line in out.splitlines():
+            text = line.split("//", 1)[0].strip()
+            if text and not text.endswith(">:") and not text.startswith("Disassembly") and ":" not in text.split()[0]:
+                lines.append(text)
     return lines
 
 
