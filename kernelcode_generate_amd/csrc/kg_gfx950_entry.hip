@@ -675,7 +675,8 @@ int launch_gemm_f32_splitk(const Mem& out, const Mem& lhs, const Mem& rhs, const
 //   256x1024x1024 13.4 / 11.5, 2x65x8001 27.5 / 23.6, and of two rounds 128x2432x1728 36 / 29.
 //   (Narrower outputs gain as much: 64x64x8192 takes half the time here. The line at 16 blocks is not
 //   where the kernels meet; it keeps the 64 x 96 output of K = 4096 that test_f32_split_k names on the
-//   32 x 32 blocks.)
+//   32 x 32 blocks. Nor is the one at 512 rows: 1024^3 would take 51 us for 77, but the fp32 cost cases
+//   name the 128 x 128-tile kernel for 1000 and 1024 rows.)
 bool gemm_skinny_pays(long long M, long long N, long long K, bool f32, bool mfma, bool splitk) {
   if (K < 64 || N < gemms::kCols) return false;  // nothing to gain: calls of a launch's length
   const long long tiles = cdiv(N, gemms::kCols);
