@@ -3,7 +3,7 @@
 // mask), 16-bit calls of other head dims (multiples of 8, causal or not), and fp32 calls
 // (fa_split_f32_kernel below).
 //
-// Such a call reads K and V once and does little else, so what bounds it is how much of the
+// A decoding step reads K and V once and does little else, so what bounds it is how much of the
 // chip keeps loads in flight. fa_fwd_mfma_kernel gives a (b,h) one workgroup (B H = 128: half
 // the CUs, 3.4 TB/s) whose K/V tiles wait for each other at barriers; here a (b,h)'s keys are
 // split over workgroups until there are two per CU, and each wave walks its own steps of keys

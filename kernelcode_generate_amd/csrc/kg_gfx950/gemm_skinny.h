@@ -7,7 +7,7 @@
 // K needs neither an LDS ring nor barriers. The k-rows of one column are put together by
 // v_perm_b32 (16-bit), and the two columns of a lane go to two v_mfma_f32_16x16x32 (fp32: to
 // 2 x 8 of 16x16x4). One LDS sum over the 16 waves, by halves, ends the call: no fp32 partials
-// in HBM and no second launch, so it also runs under graph capture. Neighbouring workgroups,
+// in HBM and no second launch. Neighbouring workgroups,
 // which share the 128-byte lines of rhs rows (and, of more rows, all of rhs), run on one XCD,
 // whose L2 fetches each line once. Pieces of 64 k, not 32, read whole lines of 16-bit lhs rows.
 //
